@@ -79,6 +79,39 @@ def test_batched_equals_single_columns(ctx, orc, qt, M, K, ncol):
         ctx.free(b)
 
 
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,nb,ncol", [(1, 1, 2), (15, 2, 4), (17, 3, 16), (129, 2, 5), (70, 5, 9), (33, 9, 12),
+                                       (300, 15, 13), (4100, 17, 2), (50, 33, 16), (31, 49, 8), (16, 64, 3),
+                                       (40, 65, 2)])
+def test_batched_edges_equal_single_columns(ctx, orc, qt, M, nb, ncol):
+    """Row counts off the 16-row tiles, K of 1 to 65 super-blocks (partial
+    slabs of 16; past 64 one vector at a time), rows that start 2-byte aligned
+    (odd Q6_K widths), every group count of 4 vectors: each column equals its
+    one-vector DMMV (to the summation floor where that runs the streaming
+    kernel, or the lane-per-block kernel of Q6_K widths off 8 super-blocks
+    or past 48, which sum in another order)."""
+    K = 256 * nb
+    print(f"batched edges q{qt} {M}x{K} cols {ncol}", flush=True)
+    W = orc.synth_tensor(qt | 0x100 if qt == 12 else qt, M, K, 91 + ncol, 1)
+    X = np.stack([orc.synth_normal_f32(K, 92, 10 + v) for v in range(ncol)])
+    Wb, Xb, Yb = ctx.upload(W), ctx.upload(X), ctx.alloc(4 * M * ncol)
+    loose = _ring(qt, K) or (qt == 14 and (nb % 8 != 0 or nb > 48)) or nb > 64 or M % 2 == 1  # (odd rows: the team kernel)
+    ctx.dmmv_batched(qt, Wb, 0, Xb, 0, Yb, 0, M, K, ncol)
+    Y = Yb.download(np.float32, M * ncol).reshape(ncol, M)
+    for v in range(ncol):
+        ref = _single(ctx, qt, Wb, X[v], M, K)
+        mag = orc.dmmv_absdot(W, qt, X[v], M, K) if loose else None
+        assert _same(Y[v], ref, mag, loose), (v, np.abs(Y[v] - ref).max())
+    if qt == 12:  # the same matrix as gate and up: silu(g) * g
+        ctx.dmmv_fused_gate_up_swiglu_batched(qt, Wb, 0, Wb, 0, Xb, 0, Yb, 0, M, K, ncol)
+        S = Yb.download(np.float32, M * ncol).reshape(ncol, M)
+        ref = orc.swiglu(Y.ravel(), Y.ravel()).reshape(ncol, M)
+        # expf and the division: a few f32 ulps of the result
+        assert np.allclose(S, ref, rtol=1e-6, atol=1e-7 * np.abs(ref).max()), np.abs(S - ref).max()
+    for b in (Wb, Xb, Yb):
+        ctx.free(b)
+
+
 def test_batched_lm_head_shape(ctx, orc):
     """The LM-head shape (M >= 65536: the one-vector path is the lane-per-block
     kernel, so the columns are held to the oracle bar only)."""

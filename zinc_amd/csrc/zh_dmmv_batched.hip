@@ -1,5 +1,7 @@
 // zh_dmmv_batched.hip -- batched decode DMMV: the Q4_K and Q6_K tile kernels
-// over several activation vectors (a skinny GEMM, recordBatchDispatchPush
+// over 2 or 4 activation vectors, for the small matrices where one launch
+// beats the two of the matrix-unit kernels (zh_dmmv_mfma.hip), and the choice
+// between them (a skinny GEMM, recordBatchDispatchPush
 // dmmv.zig:880-925 / dmmv_q4k_batch.comp, dmmv_q6k_batch.comp). Each weight
 // tile is read from HBM once and staged in LDS; the lane that owns a
 // super-block meets every vector's LDS image, so the weight stream is shared
@@ -332,13 +334,13 @@ constexpr uint32_t TILE_LDS_MAX = 163840 - 2048;
 template <int TL>
 static int launch_q4k_nv(zh_ctx *c, const LpbP &p, const LpbB &bt, uint32_t wgs, uint32_t lds) {
 #define Q4T(MM, NN) hipLaunchKernelGGL((k_dmmv_q4k_tile_nv<TL, MM, NN>), dim3(wgs), dim3(LPB_T), lds, c->stream, p, bt)
-    if (p.mode == LPB_GATE_UP) {
-        if (bt.nv == 4) Q4T(LPB_GATE_UP, 4);
-        else Q4T(LPB_GATE_UP, 2);
-    } else {
-        if (bt.nv == 4) Q4T(LPB_PLAIN, 4);
-        else Q4T(LPB_PLAIN, 2);
-    }
+    if (bt.nv == 4) {
+        if constexpr (TL <= 8) {  // (K <= 2048: tile_pays)
+            if (p.mode == LPB_GATE_UP) Q4T(LPB_GATE_UP, 4);
+            else Q4T(LPB_PLAIN, 4);
+        }
+    } else if (p.mode == LPB_GATE_UP) Q4T(LPB_GATE_UP, 2);
+    else Q4T(LPB_PLAIN, 2);
 #undef Q4T
     ZH_LAUNCH_CHECK(c);
     return ZH_OK;
@@ -346,10 +348,10 @@ static int launch_q4k_nv(zh_ctx *c, const LpbP &p, const LpbB &bt, uint32_t wgs,
 
 // Q4_K: team of <= 64 lanes (K <= 16384), 16-byte aligned matrices, every
 // segment but the last a whole number of batches, NV images + tile in LDS.
-// -1: this vector count does not fit (the caller tries fewer).
+// -1: not on the tile kernels.
 static int try_q4k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M, const LpbB &bt) {
     const uint32_t nb = p.K / 256;
-    if (nb > 64 || (bt.nv != 2 && bt.nv != 4)) return -1;
+    if (nb > 64 || (bt.nv != 2 && (bt.nv != 4 || nb > 8))) return -1;
     const uint32_t TL = pow2ceil(nb < 4 ? 4 : nb);
     const uint32_t nm = p.mode == LPB_GATE_UP ? 2 : 1;
     const uint32_t rpb = LPB_T / TL / nm;
@@ -376,10 +378,12 @@ static int try_q4k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M
 template <int TL>
 static int launch_q6k_nv(zh_ctx *c, const LpbP &p, const LpbB &bt, uint32_t wgs, uint32_t lds, uint32_t nch) {
     switch (nch) {
-#define Q6T(N)                                                                                                  \
-    case N:                                                                                                     \
-        if (bt.nv == 4) hipLaunchKernelGGL((k_dmmv_q6k_tile_nv<TL, N, 4>), dim3(wgs), dim3(LPB_T), lds, c->stream, p, bt); \
-        else hipLaunchKernelGGL((k_dmmv_q6k_tile_nv<TL, N, 2>), dim3(wgs), dim3(LPB_T), lds, c->stream, p, bt);           \
+#define Q6T(N)                                                                                                            \
+    case N:                                                                                                               \
+        if (bt.nv == 4) {                                                                                                 \
+            if constexpr (TL == 16)                                                                                       \
+                hipLaunchKernelGGL((k_dmmv_q6k_tile_nv<TL, N, 4>), dim3(wgs), dim3(LPB_T), lds, c->stream, p, bt);        \
+        } else hipLaunchKernelGGL((k_dmmv_q6k_tile_nv<TL, N, 2>), dim3(wgs), dim3(LPB_T), lds, c->stream, p, bt);         \
         break;
     Q6T(4) Q6T(5) Q6T(6) Q6T(7)  // RPB * K/256 is in (64, 128], so a tile is 3.3 .. 6.6 x 4 KB
 #undef Q6T
@@ -390,10 +394,10 @@ static int launch_q6k_nv(zh_ctx *c, const LpbP &p, const LpbB &bt, uint32_t wgs,
 }
 
 // Q6_K: rows a multiple of 16 bytes (K % 2048 == 0), team of <= 128 lanes
-// (K <= 16384), NV images + tile in LDS; tall matrices (the LM head) too.
+// (K <= 16384), NV images + tile in LDS. -1: not on the tile kernels.
 static int try_q6k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M, const LpbB &bt) {
     const uint32_t nb = p.K / 256, row_bytes = nb * 210;
-    if (row_bytes % 16 || nb > 64 || (bt.nv != 2 && bt.nv != 4)) return -1;
+    if (row_bytes % 16 || nb > 64 || (bt.nv != 2 && (bt.nv != 4 || nb != 8))) return -1;
     const uint32_t TL = pow2ceil(2 * nb < 4 ? 4 : 2 * nb);
     const uint32_t rpb = LPB_T / TL;
     const uint32_t lds = bt.nv * nb * (XB_STRIDE + 96) + rpb * row_bytes;
@@ -404,9 +408,7 @@ static int try_q6k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M
     uint32_t wgs = nbatch, cap = (uint32_t)c->cu_count;  // compiled for one workgroup per CU
     if (wgs > cap) wgs = cap;
     const uint32_t nch = (rpb * row_bytes + 4095) / 4096;
-    switch (TL) {
-    case 4: return launch_q6k_nv<4>(c, p, bt, wgs, lds, nch);
-    case 8: return launch_q6k_nv<8>(c, p, bt, wgs, lds, nch);
+    switch (TL) {  // (nb a multiple of 8)
     case 16: return launch_q6k_nv<16>(c, p, bt, wgs, lds, nch);
     case 32: return launch_q6k_nv<32>(c, p, bt, wgs, lds, nch);
     case 64: return launch_q6k_nv<64>(c, p, bt, wgs, lds, nch);
@@ -414,35 +416,52 @@ static int try_q6k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M
     }
 }
 
-// Batched DMMV on the tile kernels: y[s * n_vec + v] (= or +=) W[s] x_v for
-// v < n_vec, x_v = x[v] (f32, with the optional fused RMSNorm) or xq[v] (XQ;
-// x == nullptr). Vectors go in launches of 4 or 2 (the widest whose LDS
-// images fit beside the weight tile); a single vector left over takes the
-// one-vector path. Per vector the arithmetic is that of the one-vector tile
-// kernel, so every output equals its single-vector DMMV bit for bit.
+// Whether a launch of 2 or 4 vectors on the tile kernels beats the matrix-unit
+// kernels' two launches (about 8 us together however small the matrix; the
+// tile kernels 5.4 us, but their arithmetic grows with every vector).
+// Measured, tile / matrix units: 2 vectors of Q4_K 4096 x 4096 7.4 / 8.3 us,
+// 1024 x 12288 12.1 / 12.9, 24576 x 2048 9.9 / 12.0, and the other way
+// 24576 x 4096 18.3 / 17.3, 4096 x 12288 19.2 / 13.2; 4 vectors of
+// 4096 x 1024 7.7 / 8.2, and the other way 4096 x 4096 11.0 / 8.4, 24576 x
+// 1024 11.5 / 10.4 us. Q6_K 2048 wide alike (7.9 / 9.2); Q6_K rows
+// of no multiple of 2048 are off the tile kernels. Three vectors are two tile launches (9.3 / 8.1).
+static bool tile_pays(uint32_t nv, uint32_t rows, uint32_t K) {
+    const uint64_t n = (uint64_t)rows * K;
+    if (nv == 2) return K > 4096 ? n < 1ull << 25 : n < 1ull << 26;
+    return nv == 4 && K <= 2048 && rows < 16384;
+}
+
+// Batched DMMV: y[s * n_vec + v] (= or +=) W[s] x_v for v < n_vec, x_v = x[v]
+// (f32, with the optional fused RMSNorm) or xq[v] (XQ; x == nullptr): all
+// vectors on the matrix units (zh_dmmv_mfma.hip), or 2 or 4 on the tile
+// kernels where those are faster; a single vector, and shapes outside both,
+// one vector at a time. Per vector the arithmetic is that of the one-vector
+// tile kernel on every path, so every output equals its single-vector DMMV
+// bit for bit.
 int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const uint8_t *const *W, const uint8_t *W2,
                      const uint32_t *M, uint32_t K, uint32_t n_vec, const float *const *x, const void *const *xq,
                      float *const *y, const float *norm_w, float eps, uint32_t acc) {
     if (!zhk_lpb_supported(qtype, K) || (mode == LPB_GATE_UP && qtype != ZH_Q4_K) || nseg < 1 || nseg > 3 ||
         n_vec == 0 || (!x && !xq))
         return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "batched dmmv: unsupported qtype/K/mode/vectors");
-    uint32_t v0 = 0;
-    while (v0 < n_vec) {
+    LpbP p = {};
+    p.norm_w = norm_w; p.eps = eps;
+    p.K = K; p.acc = acc; p.nseg = nseg; p.mode = (uint32_t)mode;
+    p.row_bytes = zh_tensor_bytes(qtype, 1, K);
+    uint32_t end = 0;
+    for (uint32_t s = 0; s < nseg; s++) {
+        p.segW[s] = W[s];
+        end += M[s];
+        p.seg_end[s] = end;
+    }
+    p.segW2 = W2;
+    p.M = end;
+    const bool mfma = zhk_dmmv_mfma_fits(qtype, mode, nseg, W, W2, M, K);
+    const uint32_t rows = end * (mode == LPB_GATE_UP ? 2 : 1);
+    for (uint32_t v0 = 0; v0 < n_vec;) {
         const uint32_t left = n_vec - v0;
-        uint32_t done = 0;
-        for (uint32_t nv = left >= 4 ? 4u : left >= 2 ? 2u : 0u; nv >= 2 && !done; nv /= 2) {
-            LpbP p = {};
-            p.norm_w = norm_w; p.eps = eps;
-            p.K = K; p.acc = acc; p.nseg = nseg; p.mode = (uint32_t)mode;
-            p.row_bytes = zh_tensor_bytes(qtype, 1, K);
-            uint32_t end = 0;
-            for (uint32_t s = 0; s < nseg; s++) {
-                p.segW[s] = W[s];
-                end += M[s];
-                p.seg_end[s] = end;
-            }
-            p.segW2 = W2;
-            p.M = end;
+        if (left > 1 && (!mfma || tile_pays(left, rows, K))) {
+            const uint32_t nv = left >= 4 && K <= 2048 ? 4u : 2u;
             LpbB bt = {};
             bt.nv = nv;
             for (uint32_t v = 0; v < nv; v++) {
@@ -452,17 +471,25 @@ int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const u
             }
             const int rc = qtype == ZH_Q4_K ? try_q4k_nv(c, p, nseg, M, bt) : try_q6k_nv(c, p, nseg, M, bt);
             if (rc > 0) return rc;
-            if (rc == 0) done = nv;
+            if (rc == 0) {
+                v0 += nv;
+                continue;
+            }
         }
-        if (!done) {  // one vector
-            float *yv[3];
-            for (uint32_t s = 0; s < nseg; s++) yv[s] = y[s * n_vec + v0];
-            const int rc = zhk_dmmv_lpb(c, qtype, mode, nseg, W, W2, yv, M, x ? x[v0] : nullptr, norm_w, eps, nullptr,
-                                        K, acc, x ? nullptr : xq[v0]);
+        // (two vectors of a small Q6_K matrix off the tile kernels: one by one, 7.6 us against 9.0)
+        if (mfma && left > 1 && !(left == 2 && tile_pays(2, rows, K))) {
+            const int rc = zhk_dmmv_mfma(c, qtype, mode, nseg, W, W2, M, K, left, x ? x + v0 : nullptr,
+                                         x ? nullptr : xq + v0, y + v0, n_vec, norm_w, eps, acc);
             if (rc) return rc;
-            done = 1;
+            v0 += left;
+            continue;
         }
-        v0 += done;
+        float *yv[3];
+        for (uint32_t s = 0; s < nseg; s++) yv[s] = y[s * n_vec + v0];
+        const int rc = zhk_dmmv_lpb(c, qtype, mode, nseg, W, W2, yv, M, x ? x[v0] : nullptr, norm_w, eps, nullptr, K,
+                                    acc, x ? nullptr : xq[v0]);
+        if (rc) return rc;
+        v0++;
     }
     return ZH_OK;
 }

@@ -63,6 +63,36 @@ def test_batch_matches_single_sequences(ctx, n_seq):
     base.deinit()
 
 
+@pytest.mark.parametrize("n_seq,prefill,heads,paged", [(2, 1, 8, False), (5, 255, 16, True), (16, 130, 8, True),
+                                                       (3, 1000, 2, False), (17, 63, 4, False)])
+def test_batch_attention_edges(ctx, n_seq, prefill, heads, paged):
+    """Chunks per sequence from 64 (2 sequences) to 1 (17: two launches), the
+    new token at a page's and a chunk's first row, 1 to 8 q heads per kv head,
+    each sequence's own shuffled page table: tokens and logits as alone."""
+    import zinc_amd
+    print(f"batch attention n={n_seq} at {prefill} heads {heads} paged {paged}", flush=True)
+    cfg = dict(CFG, n_layers=2, hidden=1024, n_heads=heads, max_ctx=1024, vocab=1024)
+    base = zinc_amd.InferenceEngine(ctx, cfg)
+    engines = [base] + [base.share(ctx) for _ in range(n_seq - 1)]
+    rng = np.random.default_rng(n_seq)
+    prompts = rng.integers(0, cfg["vocab"], (n_seq, 2)).astype(np.uint32)
+    solo, logits = [], []
+    for v, e in enumerate(engines):
+        if paged:
+            e.set_pages(rng.permutation(cfg["max_ctx"] // 16))
+        e.prefill_kv_random(prefill, 300 + v)
+        solo.append(e.generate(prompts[v].tolist(), 6, start_pos=prefill))
+        logits.append(e.logits())
+        e.prefill_kv_random(prefill, 300 + v)
+    assert zinc_amd.InferenceEngine.generate_batch(engines, prompts, 6, start_pos=prefill) == solo
+    for v, e in enumerate(engines):
+        lg = e.logits()
+        assert np.allclose(lg, logits[v], rtol=1e-3, atol=1e-4 + 1e-3 * np.abs(logits[v]).max()), v
+    for e in engines[1:]:
+        e.deinit()
+    base.deinit()
+
+
 def test_batch_rejects_foreign_engines(ctx):
     import zinc_amd
     a = zinc_amd.InferenceEngine(ctx, dict(CFG, n_layers=2))

@@ -1358,39 +1358,27 @@ static int record_step_batch(zh_engine *const *es, uint32_t n, bool collect) {
                                  ys.data(), Wf(y.attn_norm), m.eps, 0));
             i0 = i1;
         }
-        // attention over each sequence's own KV cache: up to 4 sequences per
-        // launch (grid z = sequence) when they share a 1-4 q-head group,
-        // else one launch each (forking the sequences onto auxiliary streams,
-        // joined before O, measured slower than in-order launches)
-        bool all_ident = true;  // the several-sequence kernel reads identity page tables only
+        // attention over each sequence's own KV cache and page table, up to
+        // ZH_ATTN_MAXZ sequences per launch (grid z = sequence; forking the
+        // sequences onto auxiliary streams, joined before O, measured slower)
+        bool all_ident = true;
         for (uint32_t v = 0; v < n; v++) all_ident = all_ident && es[v]->pages_ident;
-        if (m.n_heads / m.n_kv_heads <= 4 && all_ident) {
-            for (uint32_t v0 = 0; v0 < n; v0 += 4) {
-                const uint32_t nz = n - v0 < 4 ? n - v0 : 4;
-                const float *aq[4], *ak[4], *av[4];
-                uint16_t *akc[4], *avc[4];
-                float *aout[4], *apart[4];
-                void *axq[4];
-                const uint32_t *apos[4];
-                for (uint32_t z = 0; z < nz; z++) {
-                    zh_engine *ev = es[v0 + z];
-                    aq[z] = ev->q; ak[z] = ev->k; av[z] = ev->v;
-                    akc[z] = ev->L[l].kc; avc[z] = ev->L[l].vc;
-                    aout[z] = ev->attn; axq[z] = ev->xq_q; apart[z] = ev->fd_part; apos[z] = ev->st + ST_POS;
-                }
-                ERC(zhk_attn_decode_fused_z(c, nz, aq, ak, av, Wf(y.q_norm), Wf(y.k_norm), e0->rope_cs, akc, avc,
-                                            e0->pages, e0->n_pages, m.max_ctx, aout, axq, m.n_heads, m.n_kv_heads,
-                                            apos, m.max_ctx, scale, m.eps, apart));
+        for (uint32_t v0 = 0; v0 < n; v0 += ZH_ATTN_MAXZ) {
+            const uint32_t nz = n - v0 < ZH_ATTN_MAXZ ? n - v0 : ZH_ATTN_MAXZ;
+            const float *aq[ZH_ATTN_MAXZ], *ak[ZH_ATTN_MAXZ], *av[ZH_ATTN_MAXZ];
+            uint16_t *akc[ZH_ATTN_MAXZ], *avc[ZH_ATTN_MAXZ];
+            float *aout[ZH_ATTN_MAXZ], *apart[ZH_ATTN_MAXZ];
+            void *axq[ZH_ATTN_MAXZ];
+            const uint32_t *apos[ZH_ATTN_MAXZ], *apg[ZH_ATTN_MAXZ];
+            for (uint32_t z = 0; z < nz; z++) {
+                zh_engine *ev = es[v0 + z];
+                aq[z] = ev->q; ak[z] = ev->k; av[z] = ev->v;
+                akc[z] = ev->L[l].kc; avc[z] = ev->L[l].vc; apg[z] = ev->pages;
+                aout[z] = ev->attn; axq[z] = ev->xq_q; apart[z] = ev->fd_part; apos[z] = ev->st + ST_POS;
             }
-        } else {
-            for (uint32_t v = 0; v < n; v++) {
-                zh_engine *ev = es[v];
-                const Layer &yv = ev->L[l];
-                zh_pos_src pos{0, ev->st + ST_POS};
-                ERC(zhk_attn_decode_fused(c, ev->q, ev->k, ev->v, Wf(y.q_norm), Wf(y.k_norm), ev->rope_cs, yv.kc,
-                                          yv.vc, ev->pages, ev->n_pages, m.max_ctx, ev->attn, ev->xq_q, m.n_heads,
-                                          m.n_kv_heads, pos, m.max_ctx, scale, m.eps, ev->fd_part, ev->pages_ident));
-            }
+            ERC(zhk_attn_decode_fused_z(c, nz, aq, ak, av, Wf(y.q_norm), Wf(y.k_norm), e0->rope_cs, akc, avc, apg,
+                                        e0->n_pages, m.max_ctx, aout, axq, m.n_heads, m.n_kv_heads, apos, m.max_ctx,
+                                        scale, m.eps, apart, all_ident));
         }
         // O (+ residual) on each sequence's XQ attention output
         const uint8_t *wo = W(y.wo), *wg = W(y.gate), *wd = W(y.down);

@@ -215,32 +215,6 @@ __global__ __launch_bounds__(AD_T, 1) void k_attn_decode(AttnP p) {
 }
 
 
-// Several sequences in one launch (batched decode): blockIdx.z selects the
-// sequence, whose buffers replace those of p0 (the weights, RoPE table and
-// geometry are shared; the sequences are at the same position).
-constexpr int AD_MAXZ = 4;
-struct AttnZ {
-    const float *q[AD_MAXZ], *k_new[AD_MAXZ], *v_new[AD_MAXZ];
-    uint16_t *kc[AD_MAXZ], *vc[AD_MAXZ];
-    const uint32_t *pos[AD_MAXZ];
-    float *part[AD_MAXZ], *out[AD_MAXZ];
-    uint32_t *counters[AD_MAXZ];
-    uint8_t *xq[AD_MAXZ];
-};
-template <int G, int TW>
-__global__ __launch_bounds__(AD_T, 1) void k_attn_decode_z(AttnP p0, AttnZ z) {
-    constexpr bool FUSED = true;
-    constexpr int MODE = AD_IDENT;
-    AttnP p = p0;
-    {
-        const uint32_t s = blockIdx.z;
-        p.q = z.q[s]; p.k_new = z.k_new[s]; p.v_new = z.v_new[s];
-        p.kc = z.kc[s]; p.vc = z.vc[s]; p.pos.dev = z.pos[s];
-        p.part = z.part[s]; p.out = z.out[s]; p.counters = z.counters[s]; p.xq = z.xq[s];
-    }
-#include "zh_attn_body.inc"
-}
-
 #include "zh_attn_ring.inc"
 
 // partials: zhk_flash_decode_partials_bytes(nh, nkv, hd, max_seq) bytes; the
@@ -348,45 +322,32 @@ int zhk_attn_decode_fused(zh_ctx *c, const float *q, const float *k, const float
     return zhk_attn_ring(c, p, nkv, max_seq, true);
 }
 
-// zhk_attn_decode_fused for n <= 4 sequences at one position in one launch
-// (grid z = sequence), identity pages, the no-wait merge. Array arguments hold
-// one entry per sequence; the weights, RoPE table and page table are shared.
+// zhk_attn_decode_fused for n <= ZH_ATTN_MAXZ sequences in one launch of the
+// ring kernel (grid z = sequence), the no-wait merge. Array arguments hold one
+// entry per sequence; the weights and RoPE table are shared. The chunks per
+// kv head shrink with n so that all sequences' chunks fill the device once:
+// with 8 sequences at a 4K context a workgroup streams 1024 tokens (8 x 16.8
+// MB of K/V per layer in 32 us = 4.2 TB/s; the register-pipelined kernel with 22 chunks
+// of 192 tokens per head and sequence, 4 sequences to a launch, took 2 x 31).
 int zhk_attn_decode_fused_z(zh_ctx *c, uint32_t n, const float *const *q, const float *const *k,
                             const float *const *v, const float *qw, const float *kw, const float *rope_cs,
-                            uint16_t *const *kc, uint16_t *const *vc, const uint32_t *pages, uint32_t n_pages,
+                            uint16_t *const *kc, uint16_t *const *vc, const uint32_t *const *pages, uint32_t n_pages,
                             uint32_t cache_tokens, float *const *out, void *const *xq_out, uint32_t nh, uint32_t nkv,
                             const uint32_t *const *pos_dev, uint32_t max_seq, float scale, float eps,
-                            float *const *partials) {
-    const uint32_t G = nkv ? nh / nkv : 0;
-    if (n == 0 || n > (uint32_t)AD_MAXZ || G == 0 || G > 4 || (G & (G - 1)))
-        return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "batched attention: %u sequences, group %u", n, G);
+                            float *const *partials, bool ident) {
+    if (n == 0 || n > ZH_ATTN_MAXZ || nkv == 0)
+        return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "batched attention: %u sequences", n);
     AttnP p = {};
-    p.q_norm = qw; p.k_norm = kw; p.rope_cs = rope_cs; p.pages = pages; p.n_pages = n_pages;
+    p.q_norm = qw; p.k_norm = kw; p.rope_cs = rope_cs; p.n_pages = n_pages;
     p.cache_tokens = cache_tokens; p.pos = zh_pos_src{0, pos_dev[0]}; p.scale = scale; p.eps = eps; p.nq = nh;
-    p.nd = attn_nd(nkv, c->cu_count);
-    p.no_wait = 1;  // chunks of other sequences share the device: no merger waits
-    p.ctl = c->err_dev;
-    const uint32_t tw = max_seq <= 8192 ? 24u : 32u;
-    p.n_chunks = attn_n_chunks(max_seq, p.nd, AD_W * tw);
-    if (p.n_chunks > p.nd) p.n_chunks = p.nd;
+    p.ident = ident ? 1u : 0u;
     AttnZ z = {};
     for (uint32_t s = 0; s < n; s++) {
-        z.q[s] = q[s]; z.k_new[s] = k[s]; z.v_new[s] = v[s]; z.kc[s] = kc[s]; z.vc[s] = vc[s];
+        z.q[s] = q[s]; z.k_new[s] = k[s]; z.v_new[s] = v[s]; z.kc[s] = kc[s]; z.vc[s] = vc[s]; z.pages[s] = pages[s];
         z.pos[s] = pos_dev[s]; z.part[s] = partials[s]; z.out[s] = out[s]; z.xq[s] = (uint8_t *)xq_out[s];
         z.counters[s] = attn_counters(partials[s], nh, nkv, FD_HD, max_seq);
     }
-    dim3 grid(nkv, p.n_chunks, n);
-#define AZ(GG)                                                                                                   \
-    if (tw == 24) hipLaunchKernelGGL((k_attn_decode_z<GG, 24>), grid, dim3(AD_T), 0, c->stream, p, z);           \
-    else hipLaunchKernelGGL((k_attn_decode_z<GG, 32>), grid, dim3(AD_T), 0, c->stream, p, z)
-    switch (G) {
-    case 1: AZ(1); break;
-    case 2: AZ(2); break;
-    default: AZ(4); break;
-    }
-#undef AZ
-    ZH_LAUNCH_CHECK(c);
-    return ZH_OK;
+    return zhk_attn_ring_z(c, p, z, n, nkv, max_seq);
 }
 
 extern "C" int zh_flash_decode(zh_ctx *c, const zh_buf *q, const zh_buf *kc, const zh_buf *vc, const zh_buf *pages,

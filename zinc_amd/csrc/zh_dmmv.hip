@@ -1257,20 +1257,10 @@ ZH_DEV uint32_t blk_bytes(uint32_t t) {
     return t == ZH_Q4_K ? 144 : t == ZH_Q5_K ? 176 : t == ZH_Q6_K ? 210 : t == ZH_Q8_0 ? 34 : t == ZH_MXFP4 ? 17 : t == ZH_F16 ? 2 : 4;
 }
 
-__global__ void k_dequant(uint32_t qtype, const uint8_t *__restrict__ W, uint32_t row0, uint32_t n_rows,
-                          uint32_t K, float *__restrict__ out, const uint32_t *row_from_dev, uint32_t clamp_rows,
-                          uint32_t gather) {
-    uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t rr = blockIdx.y;
-    if (e >= K || rr >= n_rows) return;
-    uint32_t row = row0 + rr;
-    if (row_from_dev) {
-        // one id and consecutive rows, or (gather) one id per output row
-        row = gather ? row_from_dev[rr] : row_from_dev[0] + rr;
-        if (row >= clamp_rows) row = clamp_rows - 1;  // embedToken safe_id clamp (forward.zig:4271)
-    }
+// Element e of row `row` (dequantRow's f32 value).
+ZH_DEV float dequant_at(uint32_t qtype, const uint8_t *__restrict__ W, uint64_t row, uint32_t K, uint32_t e) {
     uint64_t rb = (uint64_t)(K / blk_elems(qtype)) * blk_bytes(qtype);
-    const uint8_t *r = W + (uint64_t)row * rb;
+    const uint8_t *r = W + row * rb;
     float v = 0.f;
     switch (qtype) {
     case ZH_Q4_K: {
@@ -1326,7 +1316,47 @@ __global__ void k_dequant(uint32_t qtype, const uint8_t *__restrict__ W, uint32_
     case ZH_F16: v = h2f(((const uint16_t *)r)[e]); break;
     case ZH_F32: v = ((const float *)r)[e]; break;
     }
-    out[(size_t)rr * K + e] = v;
+    return v;
+}
+
+__global__ void k_dequant(uint32_t qtype, const uint8_t *__restrict__ W, uint32_t row0, uint32_t n_rows,
+                          uint32_t K, float *__restrict__ out, const uint32_t *row_from_dev, uint32_t clamp_rows,
+                          uint32_t gather) {
+    uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t rr = blockIdx.y;
+    if (e >= K || rr >= n_rows) return;
+    uint32_t row = row0 + rr;
+    if (row_from_dev) {
+        // one id and consecutive rows, or (gather) one id per output row
+        row = gather ? row_from_dev[rr] : row_from_dev[0] + rr;
+        if (row >= clamp_rows) row = clamp_rows - 1;  // embedToken safe_id clamp (forward.zig:4271)
+    }
+    out[(size_t)rr * K + e] = dequant_at(qtype, W, row, K, e);
+}
+
+// One row for each of up to 16 sequences: row id[s][0] to out[s] (blockIdx.y = s).
+struct DequantZ {
+    const uint32_t *id[16];
+    float *out[16];
+};
+__global__ void k_dequant_z(uint32_t qtype, const uint8_t *__restrict__ W, uint32_t K, uint32_t clamp_rows, DequantZ z) {
+    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x, s = blockIdx.y;
+    if (e >= K) return;
+    z.out[s][e] = dequant_at(qtype, W, min(z.id[s][0], clamp_rows - 1), K, e);
+}
+int zhk_dequant_rows_z(zh_ctx *c, uint32_t qtype, const uint8_t *W, uint32_t K, uint32_t n, const uint32_t *const *ids,
+                       uint32_t clamp_rows, float *const *out) {
+    for (uint32_t v0 = 0; v0 < n; v0 += 16) {
+        const uint32_t nz = n - v0 < 16 ? n - v0 : 16;
+        DequantZ z = {};
+        for (uint32_t s = 0; s < nz; s++) {
+            z.id[s] = ids[v0 + s];
+            z.out[s] = out[v0 + s];
+        }
+        hipLaunchKernelGGL(k_dequant_z, dim3((K + 255) / 256, nz), dim3(256), 0, c->stream, qtype, W, K, clamp_rows, z);
+        ZH_LAUNCH_CHECK(c);
+    }
+    return ZH_OK;
 }
 
 int zhk_dequant_rows(zh_ctx *c, uint32_t qtype, const uint8_t *W, uint32_t row0, uint32_t n_rows, uint32_t K,

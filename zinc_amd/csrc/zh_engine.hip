@@ -123,7 +123,7 @@ static uint64_t align256(uint64_t x) { return (x + 255) & ~255ull; }
 // ---------------------------------------------------------------------------
 // Small kernels owned by the engine.
 // ---------------------------------------------------------------------------
-__global__ void k_advance(uint32_t *st, const uint32_t *prompt) {
+ZH_DEV void advance(uint32_t *st, const uint32_t *prompt) {
     // End of a step: count the generated token, move to the next position and
     // pick the next input token (prompt while it lasts, else the argmax).
     uint32_t s = st[ST_STEP], np = st[ST_NPROMPT];
@@ -133,6 +133,7 @@ __global__ void k_advance(uint32_t *st, const uint32_t *prompt) {
     st[ST_POS] += 1;
     st[ST_TOKEN_IN] = (s < np) ? prompt[s] : st[ST_TOKEN_OUT];
 }
+__global__ void k_advance(uint32_t *st, const uint32_t *prompt) { advance(st, prompt); }
 
 // The step's greedy token and the step advance in one launch: every
 // workgroup reduces a strided share of the logits (first maximum wins) and
@@ -142,9 +143,8 @@ __global__ void k_advance(uint32_t *st, const uint32_t *prompt) {
 // (argmaxGreedy, forward.zig:10348-10356) and advances the state as
 // k_advance. The counter is left zero for the next launch.
 constexpr uint32_t TAIL_WGS = 256;  // (am_part holds 256 (value, index) pairs)
-__global__ __launch_bounds__(256) void k_argmax_advance(const float *__restrict__ x, uint32_t n, uint32_t *partials,
-                                                        uint32_t *cnt, uint32_t *ring, uint32_t *st,
-                                                        const uint32_t *prompt) {
+ZH_DEV void argmax_advance(const float *__restrict__ x, uint32_t n, uint32_t *partials, uint32_t *cnt, uint32_t *ring,
+                           uint32_t *st, const uint32_t *prompt) {
     float bv = -INFINITY;
     uint32_t bi = 0xFFFFFFFFu;
     // 4 logits per load (x is 16-byte aligned); workgroup 0 also takes the n % 4 last ones
@@ -196,6 +196,26 @@ __global__ __launch_bounds__(256) void k_argmax_advance(const float *__restrict_
         st[ST_TOKEN_IN] = (s < np) ? prompt[s] : bi;
     }
 }
+__global__ __launch_bounds__(256) void k_argmax_advance(const float *__restrict__ x, uint32_t n, uint32_t *partials,
+                                                        uint32_t *cnt, uint32_t *ring, uint32_t *st,
+                                                        const uint32_t *prompt) {
+    argmax_advance(x, n, partials, cnt, ring, st, prompt);
+}
+
+// The same tail for up to 16 sequences (blockIdx.y) in one launch: a launch
+// per sequence for the argmax's two passes and the advance cost a batched
+// step of 8 sequences 60 us more.
+constexpr uint32_t TAIL_MAXZ = 16;
+struct TailZ {
+    const float *x[TAIL_MAXZ];
+    uint32_t *partials[TAIL_MAXZ], *cnt[TAIL_MAXZ], *ring[TAIL_MAXZ], *st[TAIL_MAXZ];
+    const uint32_t *prompt[TAIL_MAXZ];
+};
+__global__ __launch_bounds__(256) void k_argmax_advance_z(TailZ z, uint32_t n) {
+    const uint32_t s = blockIdx.y;
+    argmax_advance(z.x[s], n, z.partials[s], z.cnt[s], z.ring[s], z.st[s], z.prompt[s]);
+}
+__global__ void k_advance_z(TailZ z) { advance(z.st[threadIdx.x], z.prompt[threadIdx.x]); }
 
 // Seeded N(0,1) fp16 values for logical tokens [0, n) of one layer, written
 // into the head-major cache; counter = t*kv_dim + h*head_dim + d, as the
@@ -1337,8 +1357,12 @@ static int record_step_batch(zh_engine *const *es, uint32_t n, bool collect) {
     std::vector<const float *> xs(n);
     std::vector<const void *> xqs(n);
     std::vector<float *> ys(3 * n);
-    for (uint32_t v = 0; v < n; v++)
-        ERC(zhk_dequant_rows(c, e0->embd.type, W(e0->embd), 0, 1, H, es[v]->hidden, es[v]->st + ST_TOKEN_IN, m.vocab));
+    std::vector<const uint32_t *> ids(n);
+    for (uint32_t v = 0; v < n; v++) {
+        ids[v] = es[v]->st + ST_TOKEN_IN;
+        ys[v] = es[v]->hidden;
+    }
+    ERC(zhk_dequant_rows_z(c, e0->embd.type, W(e0->embd), H, n, ids.data(), m.vocab, ys.data()));
     for (uint32_t l = 0; l < m.n_layers; l++) {
         const Layer &y = e0->L[l];
         // Q, K, V (attn_norm fused): one batched launch per run of equal types
@@ -1412,13 +1436,22 @@ static int record_step_batch(zh_engine *const *es, uint32_t n, bool collect) {
         }
         ERC(zhk_dmmv_batched(c, e0->lm.type, 0, 1, &wl, nullptr, &V, H, n, xs.data(), nullptr, ys.data(),
                              (const float *)(A + e0->out_norm.off), m.eps, 0));
-        for (uint32_t v = 0; v < n; v++)
-            ERC(zhk_argmax(c, es[v]->logits, V, es[v]->st + ST_TOKEN_OUT, es[v]->am_part, es[v]->ring,
-                           es[v]->st + ST_GEN));
     }
-    for (uint32_t v = 0; v < n; v++)
-        hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, es[v]->st, (const uint32_t *)es[v]->prompt);
-    ZH_LAUNCH_CHECK(c);
+    for (uint32_t v0 = 0; v0 < n; v0 += TAIL_MAXZ) {
+        const uint32_t nz = n - v0 < TAIL_MAXZ ? n - v0 : TAIL_MAXZ;
+        TailZ z = {};
+        for (uint32_t i = 0; i < nz; i++) {
+            zh_engine *ev = es[v0 + i];
+            z.x[i] = ev->logits; z.partials[i] = ev->am_part; z.cnt[i] = ev->am_cnt; z.ring[i] = ev->ring;
+            z.st[i] = ev->st; z.prompt[i] = ev->prompt;
+        }
+        if (collect)
+            hipLaunchKernelGGL(k_argmax_advance_z, dim3(nz > 4 ? TAIL_WGS / 4 : TAIL_WGS, nz), dim3(256), 0, c->stream, z,
+                               m.vocab);
+        else
+            hipLaunchKernelGGL(k_advance_z, dim3(1), dim3(nz), 0, c->stream, z);
+        ZH_LAUNCH_CHECK(c);
+    }
     return ZH_OK;
 }
 

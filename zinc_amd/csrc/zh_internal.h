@@ -127,6 +127,9 @@ int zhk_dmmv_moe(zh_ctx *ctx, uint32_t qtype, const uint8_t *W, uint64_t expert_
                  const uint32_t *routing, const void *xq, uint64_t xq_slot_stride, float *y,
                  uint32_t M, uint32_t K, uint32_t n_used, int gate_up, const uint8_t *W2, uint32_t n_experts,
                  uint32_t *err = nullptr);
+// Row ids[s][0] (clamped) of W to out[s] for n sequences.
+int zhk_dequant_rows_z(zh_ctx *ctx, uint32_t qtype, const uint8_t *W, uint32_t K, uint32_t n, const uint32_t *const *ids,
+                       uint32_t clamp_rows, float *const *out);
 int zhk_dequant_rows(zh_ctx *ctx, uint32_t qtype, const uint8_t *W, uint32_t row0, uint32_t n_rows,
                      uint32_t K, float *out, const uint32_t *row_from_dev, uint32_t clamp_rows, uint32_t gather = 0);
 uint32_t zh_router_shift(uint64_t K);  // the router flag's shift of zhk_synth_tensor (zh_runtime.hip)

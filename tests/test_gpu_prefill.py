@@ -216,3 +216,30 @@ def test_flash_attn_batched_matches_reference(ctx, nh, nkv, seq_start, n):
     bound = 4e-3 * np.abs(ref).reshape(n, nh, 128).max(axis=2).repeat(128, axis=1) + 1e-3
     err = np.abs(got - ref)
     assert (err <= bound).all(), (err.max(), np.unravel_index(err.argmax(), err.shape))
+
+
+@pytest.mark.parametrize("nh,nkv,seq_start,n,scale", [
+    (8, 8, 0, 1, 0.0), (8, 1, 63, 1, 0.0), (4, 2, 64, 64, 0.0), (8, 2, 127, 1, 0.0), (8, 2, 128, 1, 0.0),
+    (4, 4, 65, 63, 0.3), (2, 1, 0, 129, -0.05), (8, 4, 255, 65, 0.0), (16, 2, 500, 200, 0.0)])
+def test_flash_attn_batched_edges(ctx, nh, nkv, seq_start, n, scale):
+    """One to thirteen key blocks over the one-group and the four-group form
+    (more than 128 keys), query tiles ending inside one, groups that see no
+    key of some queries, every q-per-kv count, a given (also negative) scale.
+    The bound of test_flash_attn_batched_matches_reference."""
+    rng = np.random.default_rng(nh * 1000 + seq_start + n)
+    cache_tokens = 1024
+    pages = rng.permutation(cache_tokens // 16).astype(np.uint32)
+    k16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
+    v16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
+    q = rng.standard_normal((n, nh * 128)).astype(np.float32)
+    bufs = [ctx.upload(q), ctx.upload(k16), ctx.upload(v16), ctx.upload(pages), ctx.alloc(2 * n * nh * 128)]
+    ctx.flash_attn_batched(*bufs[:4], len(pages), cache_tokens, bufs[4], nh, nkv, 128, seq_start, n, scale)
+    ctx.sync()
+    got = bufs[4].download(np.float16, n * nh * 128).astype(np.float64).reshape(n, -1)
+    ref = _causal_ref(q, k16, v16, pages, nh, nkv, seq_start, scale or 1 / np.sqrt(128))
+    bound = 4e-3 * np.abs(ref).reshape(n, nh, 128).max(axis=2).repeat(128, axis=1) + 1e-3
+    err = np.abs(got - ref)
+    assert (err <= bound).all(), (err.max(), np.unravel_index(err.argmax(), err.shape))
+    for b in bufs:
+        ctx.free(b)
+

@@ -630,147 +630,223 @@ __global__ __launch_bounds__(256) void k_swiglu_rows_f16(const float *__restrict
 }
 
 // Causal prefill attention on the MFMA units (flash attention): workgroup =
-// one q head x AQ = 64 queries (16 per wave), key blocks of AK = 64 staged in
-// LDS (K row-major, V transposed to [d][key]). Per block each wave computes
-// S = Q K^T (16 x 64, v_mfma_f32_16x16x32_f16 over d), scales and masks it,
-// updates the running row maximum and sum (online softmax, f32), writes
-// P = exp(S - m) as fp16 to its own LDS tile (the D layout of S holds 4 rows
-// per lane; the A layout of the next product holds 8 keys of one row) and
-// accumulates O += P V (16 x 128). Q, K, V and P are fp16 operands with f32
-// accumulation. Query tiles run longest first (causal: tile t sees t + 1
-// blocks).
+// one q head x AQ = 64 queries, NG groups of two waves; group g takes key
+// blocks g, g + NG, ... of AK = 64 keys, each wave 32 queries of them, and the
+// groups' outputs are merged at the end (log-sum-exp weights in LDS). The
+// longest query tile bounds the launch (one workgroup per CU at 512 tokens),
+// so its chain of key blocks is cut by NG. Bound by LDS traffic (1.3 us of
+// the 3.7 a round of NG blocks takes) with the softmax and the MFMAs behind
+// barriers. 32 heads: 512 queries at 0 24 -> 19.4 us, 509 after 1031 tokens
+// 66.5 -> 39.7 us (44.5 with four waves of 16 queries per group, which read
+// every K and V fragment twice as often).
+//
+// Scores are taken transposed, S^T = K Q^T (tokens x queries,
+// v_mfma_f32_16x16x32_f16 over d), so a lane holds 16 tokens of one query:
+// the softmax's maximum is in-lane plus two lane-group exchanges, its sum
+// stays in the lane until the end, and the fp16 probabilities are the second
+// product's operand as they lie (O^T += V^T P^T with the keys of an MFMA step
+// taken as tokens 4 lg + r of two 16-token tiles). V stays row-major in LDS;
+// its transposed fragments come from ds_read_b64_tr_b16. (Before: P through
+// LDS in another layout, V transposed by 2-byte LDS stores, row sums by DPP
+// for every block.) Q, K, V and P are fp16 operands with f32 accumulation.
+// Query tiles run longest first (causal: tile t sees t + 1 blocks).
 constexpr int AQ = 64, AK = 64;
-constexpr int AKLD = 128 + 8;  // halfs per K row (272 B)
-constexpr int AVLD = AK + 8;   // halfs per P row (144 B)
-// V transposed, [d][key] with 64 keys per row (128 B, no padding): the 16-byte
-// chunk of keys 8c .. 8c + 7 of row d sits at chunk c ^ ((d / 8) % 8), so the
-// 16 lanes that store one key's 16 chunks of dims (2-byte stores) spread over
-// 8 bank groups instead of one, and a B fragment is still one 16-byte read
-ZH_DEV uint32_t vt_at(uint32_t d, uint32_t key) { return d * AK + ((((key >> 3) ^ (d >> 3)) & 7) << 3) + (key & 7); }
-__global__ __launch_bounds__(256) void k_attn_prefill_mfma(const float *__restrict__ q, const uint16_t *__restrict__ kc,
-                                                           const uint16_t *__restrict__ vc,
-                                                           const uint32_t *__restrict__ pages, uint32_t n_pages,
-                                                           uint32_t cache_tokens, uint32_t nq, uint32_t nkv,
-                                                           uint32_t pos0, uint32_t N, float scale,
-                                                           _Float16 *__restrict__ out) {
+constexpr int AKLD = 128 + 8;    // halfs per K row: 16 rows' 16-byte reads hit every bank once
+constexpr int AVLD = 128 + 16;   // halfs per V row: 8 rows' 32-byte pieces hit every bank once
+constexpr uint32_t AP_GROUP = (AK * (AKLD + AVLD)) * 2;  // LDS of a group (its merge rows fit in it)
+constexpr uint32_t AP_OLD = 132;                          // floats per query of a group's output
+static_assert(AQ * AP_OLD * 4 + AQ * 8 <= AP_GROUP, "the merge rows overlay the key block");
+template <int NG>
+__global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                                               const uint16_t *__restrict__ vc,
+                                                               const uint32_t *__restrict__ pages, uint32_t n_pages,
+                                                               uint32_t cache_tokens, uint32_t nq, uint32_t nkv,
+                                                               uint32_t pos0, uint32_t N, float scale,
+                                                               _Float16 *__restrict__ out) {
     constexpr int HD = 128;
-    __shared__ __align__(16) _Float16 ks[AK * AKLD];
-    __shared__ __align__(16) uint16_t vt[HD * AK];
-    __shared__ __align__(16) _Float16 pl[4][16 * AVLD];
-    const uint32_t h = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    extern __shared__ __align__(16) uint8_t lds[];
+    typedef __fp16 tr4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) tr4 lds_tr4;
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const uint32_t g = wave / 2, w2 = wave % 2, tg = tid & 127, li = lane % 16, lg = lane / 16;
+    _Float16 *const ks = (_Float16 *)(lds + g * AP_GROUP), *const vs = ks + AK * AKLD;
+    // workgroups go round robin over the XCDs: the q heads of a kv head to one
+    const uint32_t G = nq / nkv, kvh = blockIdx.x % nkv, h = kvh * G + blockIdx.x / nkv;
     const uint32_t i0 = (gridDim.y - 1 - blockIdx.y) * AQ;  // longest tiles first
-    const uint32_t kvh = h / (nq / nkv), li = lane % 16, lg = lane / 16;
     const uint16_t *kh = kc + (size_t)kvh * cache_tokens * HD;
     const uint16_t *vh = vc + (size_t)kvh * cache_tokens * HD;
-    // Q fragments (A operand): row i0 + 16 wave + li, d = 32 ks + 8 lg .. +7
-    half8 qa[4];
-    {
-        const float *qp = q + (size_t)min(i0 + 16 * wave + li, N - 1) * nq * HD + (size_t)h * HD + 8 * lg;
+    // Q fragments (B operand): query i0 + 32 w2 + 16 t + li, d = 32 k4 + 8 lg .. +7
+    half8 qa[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const float *qp = q + (size_t)min(i0 + 32 * w2 + 16 * t + li, N - 1) * nq * HD + (size_t)h * HD + 8 * lg;
 #pragma unroll
         for (int k4 = 0; k4 < 4; k4++) {
             const f32x4 a = *(const f32x4 *)(qp + 32 * k4), b = *(const f32x4 *)(qp + 32 * k4 + 4);
-            qa[k4] = half8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
-                           (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
+            qa[t][k4] = half8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
+                              (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
         }
     }
-    f32x4v o[8];
+    f32x4v o[2][8];  // O^T: dims 16 db + 4 lg + r of query 16 t + li
 #pragma unroll
-    for (int db = 0; db < 8; db++) o[db] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    float m[4], l[4];
+    for (int t = 0; t < 2; t++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) { m[r] = -INFINITY; l[r] = 0.f; }
+        for (int db = 0; db < 8; db++) o[t][db] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // base-2 running maxima (all lg alike), this lane's share of the sums
+    const float c = scale * 1.44269504088896340736f;
     const uint32_t kmax = pos0 + min(i0 + AQ, N) - 1;  // last key any query of the workgroup sees
-    const uint32_t qpos = pos0 + i0 + 16 * wave + 4 * lg;  // position of this lane's row r = 0
-    _Float16 *pw = pl[wave];
-    // the key block's K and V chunks (16 B of one key each: 4 per thread)
+    const uint32_t nblk = kmax / AK + 1, nstep = (nblk + NG - 1) / NG;
+    const uint32_t q0 = pos0 + i0 + 32 * w2;
+    // the key block's K and V chunks (16 B of one key each: 8 per thread)
     // wait in registers, requested while the previous block computes; rows
     // past kmax are loaded clamped and masked below
-    u32x4 pk[4], pv[4];
-    auto load_kv = [&](uint32_t kb) __attribute__((always_inline)) {
+    u32x4 pk[8], pv[8];
+    auto load = [&](uint32_t kb, const uint16_t *src, u32x4 (&dst)[8]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const uint32_t c = tid + 256 * it, key = c / 16, ch = c % 16, t = min(kb * AK + key, kmax);
-            uint32_t ph = pages[min(t / 16, n_pages - 1)] * 16 + t % 16;
-            ph = ph < cache_tokens ? ph : 0u;
-            pk[it] = *(const u32x4 *)(kh + (size_t)ph * HD + ch * 8);
-            pv[it] = *(const u32x4 *)(vh + (size_t)ph * HD + ch * 8);
+        for (int it = 0; it < 8; it++) {  // keys 8 it + tg / 16: one page
+            const uint32_t pg = min(kb * 4 + it / 2, kmax / 16);
+            uint32_t ph = pages[min(pg, n_pages - 1)] * 16;
+            const uint32_t row = 8 * (it & 1) + tg / 16, r = pg == kmax / 16 ? min(row, kmax % 16) : row;
+            ph = ph + 16 <= cache_tokens || ph + r < cache_tokens ? ph + r : 0u;
+            dst[it] = *(const u32x4 *)(src + (size_t)ph * HD + (tg % 16) * 8);
         }
     };
-    load_kv(0);
-    for (uint32_t kb = 0; kb * AK <= kmax; kb++) {
-        // stage the key block: K rows as they are, V transposed
+    if (g < nblk) {
+        load(g, kh, pk);
+        load(g, vh, pv);
+    }
+    for (uint32_t st = 0; st < nstep; st++) {
+        const uint32_t kb = st * NG + g;
+        const bool mine = kb < nblk;  // uniform in the group
+        if (mine) {
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const uint32_t c = tid + 256 * it, key = c / 16, ch = c % 16;
-            *(u32x4 *)(ks + key * AKLD + ch * 8) = pk[it];
-            const uint32_t w[4] = {pv[it].x, pv[it].y, pv[it].z, pv[it].w};
-#pragma unroll
-            for (int e = 0; e < 8; e++) vt[vt_at(ch * 8 + e, key)] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+            for (int it = 0; it < 8; it++) {
+                *(u32x4 *)(ks + (8 * it + tg / 16) * AKLD + (tg % 16) * 8) = pk[it];
+                *(u32x4 *)(vs + (8 * it + tg / 16) * AVLD + (tg % 16) * 8) = pv[it];
+            }
         }
         __syncthreads();
-        if ((kb + 1) * AK <= kmax) load_kv(kb + 1);
-        f32x4v sc[4];
-#pragma unroll
-        for (int jb = 0; jb < 4; jb++) {
-            sc[jb] = f32x4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k4 = 0; k4 < 4; k4++) {
-                const half8 b = *(const half8 *)(ks + (16 * jb + li) * AKLD + 32 * k4 + 8 * lg);
-                sc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[k4], b, sc[jb], 0, 0, 0);
-            }
-        }
-        float mb[4], f[4], ls[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            mb[r] = -INFINITY;
+        const bool more = kb + NG < nblk;
+        if (more) load(kb + NG, kh, pk);
+        const bool sees = mine && kb * AK <= q0 + 31;  // (uniform per wave: some query of it sees the block)
+        f32x4v sc[2][4];
+        if (sees) {
 #pragma unroll
             for (int jb = 0; jb < 4; jb++) {
-                const uint32_t key = kb * AK + 16 * jb + li;
-                const float v = key <= qpos + r ? sc[jb][r] * scale : -INFINITY;
-                sc[jb][r] = v;
-                mb[r] = fmaxf(mb[r], v);
+                sc[0][jb] = sc[1][jb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k4 = 0; k4 < 4; k4++) {
+                    const half8 a = *(const half8 *)(ks + (16 * jb + li) * AKLD + 32 * k4 + 8 * lg);
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+                        sc[t][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qa[t][k4], sc[t][jb], 0, 0, 0);
+                }
             }
-            // block 0 holds key 0, visible to every row: m is finite from then on
-            const float mn = fmaxf(m[r], row16_max(mb[r]));
-            f[r] = expf(m[r] - mn);
-            m[r] = mn;
-            ls[r] = 0.f;
         }
+        if (more) load(kb + NG, vh, pv);  // (after the scores: their registers are taken until then)
+        if (sees) {
+            const bool whole = kb * AK + AK - 1 <= q0;  // every query sees every key
+            half8 pb[2][2];
 #pragma unroll
-        for (int jb = 0; jb < 4; jb++)
+            for (int t = 0; t < 2; t++) {
+                const uint32_t qpos = q0 + 16 * t + li;
+                float mb = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float p = expf(sc[jb][r] - m[r]);
-                ls[r] += p;
-                pw[(4 * lg + r) * AVLD + 16 * jb + li] = (_Float16)p;
+                for (int jb = 0; jb < 4; jb++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        float v = sc[t][jb][r] * c;
+                        if (!whole) v = kb * AK + 16 * jb + 4 * lg + r <= qpos ? v : -INFINITY;
+                        sc[t][jb][r] = v;
+                        mb = fmaxf(mb, v);
+                    }
+                mb = xor32_max(xor16_max(mb));
+                const float mn = fmaxf(m[t], mb), ms = mn == -INFINITY ? 0.f : mn;
+                const float f = __builtin_amdgcn_exp2f(m[t] - ms);  // (m = -inf: 0)
+                m[t] = mn;
+                float ls = 0.f;
+#pragma unroll
+                for (int jb = 0; jb < 4; jb++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float p = __builtin_amdgcn_exp2f(sc[t][jb][r] - ms);
+                        ls += p;
+                        pb[t][jb >> 1][4 * (jb & 1) + r] = (_Float16)p;
+                    }
+                l[t] = fmaf(l[t], f, ls);
+#pragma unroll
+                for (int db = 0; db < 8; db++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[t][db][r] *= f;
             }
 #pragma unroll
-        for (int r = 0; r < 4; r++) l[r] = fmaf(l[r], f[r], row16_sum(ls[r]));
+            for (int s2 = 0; s2 < 2; s2++)
 #pragma unroll
-        for (int db = 0; db < 8; db++)
+                for (int db = 0; db < 8; db++) {
+                    // lane l of a 16-lane group addresses token l / 4's dims 4 (l % 4) .. +3 and
+                    // receives dim l of the four tokens
+                    _Float16 *va = vs + (32 * s2 + 4 * lg + li / 4) * AVLD + 16 * db + 4 * (li % 4);
+                    const tr4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4 *)(va));
+                    const tr4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4 *)(va + 16 * AVLD));
+                    const half8 a = {(_Float16)t0[0], (_Float16)t0[1], (_Float16)t0[2], (_Float16)t0[3],
+                                     (_Float16)t1[0], (_Float16)t1[1], (_Float16)t1[2], (_Float16)t1[3]};
 #pragma unroll
-            for (int r = 0; r < 4; r++) o[db][r] *= f[r];
-        // the wave reads back its own P tile (LDS operations of a wave complete in order)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int k2 = 0; k2 < 2; k2++) {
-            const half8 a = *(const half8 *)(pw + li * AVLD + 32 * k2 + 8 * lg);
-#pragma unroll
-            for (int db = 0; db < 8; db++) {
-                const half8 b = *(const half8 *)(vt + vt_at(16 * db + li, 32 * k2 + 8 * lg));
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, o[db], 0, 0, 0);
-            }
+                    for (int t = 0; t < 2; t++)
+                        o[t][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb[t][s2], o[t][db], 0, 0, 0);
+                }
         }
         __syncthreads();  // the block's K / V tiles are rewritten next
     }
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const uint32_t i = i0 + 16 * wave + 4 * lg + r;
-        if (i < N) {
-            const float inv = 1.0f / l[r];
-            _Float16 *op = out + (size_t)i * nq * HD + (size_t)h * HD + li;
+    for (int t = 0; t < 2; t++) l[t] = xor32_sum(xor16_sum(l[t]));
+    if constexpr (NG == 1) {
 #pragma unroll
-            for (int db = 0; db < 8; db++) op[16 * db] = (_Float16)(o[db][r] * inv);
+        for (int t = 0; t < 2; t++) {
+            const uint32_t i = i0 + 32 * w2 + 16 * t + li;
+            if (i >= N) continue;
+            const float inv = 1.0f / l[t];
+            _Float16 *op = out + (size_t)i * nq * HD + (size_t)h * HD + 4 * lg;
+#pragma unroll
+            for (int db = 0; db < 8; db++)
+                *(half4 *)(op + 16 * db) = half4{(_Float16)(o[t][db][0] * inv), (_Float16)(o[t][db][1] * inv),
+                                                 (_Float16)(o[t][db][2] * inv), (_Float16)(o[t][db][3] * inv)};
+        }
+    } else {
+        float *const go = (float *)(lds + g * AP_GROUP), *const gm = go + AQ * AP_OLD, *const gl = gm + AQ;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint32_t qr = 32 * w2 + 16 * t + li;
+#pragma unroll
+            for (int db = 0; db < 8; db++) *(f32x4v *)(go + qr * AP_OLD + 16 * db + 4 * lg) = o[t][db];
+            if (lg == 0) {
+                gm[qr] = m[t];
+                gl[qr] = l[t];
+            }
+        }
+        __syncthreads();
+        // thread: query tid / (2 NG), 64 / NG dims
+        constexpr int ND = 64 / NG;
+        const uint32_t mq = tid / (2 * NG), d0 = tid % (2 * NG) * ND, i = i0 + mq;
+        float M = -INFINITY, w[NG], L = 0.f, r[ND];
+#pragma unroll
+        for (int k = 0; k < NG; k++) M = fmaxf(M, ((float *)(lds + k * AP_GROUP))[AQ * AP_OLD + mq]);
+#pragma unroll
+        for (int d = 0; d < ND; d++) r[d] = 0.f;
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const float *ko = (const float *)(lds + k * AP_GROUP);
+            w[k] = __builtin_amdgcn_exp2f(ko[AQ * AP_OLD + mq] - M);  // (a group without keys of the query: 0)
+            L = fmaf(ko[AQ * AP_OLD + AQ + mq], w[k], L);
+#pragma unroll
+            for (int d = 0; d < ND; d++) r[d] = fmaf(ko[mq * AP_OLD + d0 + d], w[k], r[d]);
+        }
+        if (i < N) {
+            const float inv = 1.0f / L;
+            _Float16 *op = out + (size_t)i * nq * HD + (size_t)h * HD + d0;
+#pragma unroll
+            for (int d = 0; d < ND; d += 4)
+                *(half4 *)(op + d) = half4{(_Float16)(r[d] * inv), (_Float16)(r[d + 1] * inv),
+                                           (_Float16)(r[d + 2] * inv), (_Float16)(r[d + 3] * inv)};
         }
     }
 }
@@ -795,8 +871,14 @@ int zhk_attn_prefill(zh_ctx *c, const float *q, const uint16_t *kc, const uint16
                      uint32_t n_pages, uint32_t cache_tokens, uint32_t nq, uint32_t nkv, uint32_t hd, uint32_t pos0,
                      uint32_t N, float scale, _Float16 *out) {
     if (hd != 128 || nkv == 0 || nq % nkv) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "attn_prefill heads");
-    hipLaunchKernelGGL(k_attn_prefill_mfma, dim3(nq, (N + AQ - 1) / AQ), dim3(256), 0, c->stream, q, kc, vc, pages,
-                       n_pages, cache_tokens, nq, nkv, pos0, N, scale, out);
+    const dim3 grid(nq, (N + AQ - 1) / AQ);
+    // two key blocks or fewer for any query: one group
+    if (pos0 + N <= 2 * AK)
+        hipLaunchKernelGGL(k_attn_prefill_mfma<1>, grid, dim3(128), AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
+                           cache_tokens, nq, nkv, pos0, N, scale, out);
+    else
+        hipLaunchKernelGGL(k_attn_prefill_mfma<4>, grid, dim3(512), 4 * AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
+                           cache_tokens, nq, nkv, pos0, N, scale, out);
     ZH_LAUNCH_CHECK(c);
     return ZH_OK;
 }

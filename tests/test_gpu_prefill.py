@@ -80,6 +80,30 @@ def test_gemm_matches_fp16_operand_reference(ctx, orc, qtype, M, K, N):
         ctx.free(b)
 
 
+@pytest.mark.parametrize("qtype,M,K,N", [
+    (12, 24500, 512, 509), (12, 24500, 2048, 200),     # 256 tokens x 192 rows, whole and with K split
+    (12, 1000, 2304, 129), (14, 1000, 2304, 257), (14, 24500, 256, 256),  # 256 x 128, odd steps, one split
+    (12, 130, 256, 128),                                # 128 x 128
+])
+def test_gemm_tile_edges(ctx, orc, qtype, M, K, N):
+    """Every tile of the dispatch with a ragged last row and token tile,
+    accumulating: f32 sums of K / 32 matrix instructions of 32 products, each
+    addition within an ulp (2^-23) of the sum of magnitudes."""
+    raw = orc.synth_tensor(qtype, M, K, 2000 + M, N)
+    w16 = dequant_f16(orc, raw, qtype, M, K).astype(np.float64)
+    rng = np.random.default_rng(M * 5 + N)
+    x16 = rng.standard_normal((N, K)).astype(np.float16)
+    y0 = rng.standard_normal((N, M)).astype(np.float32)
+    ref = y0 + x16.astype(np.float64) @ w16.T
+    mag = np.abs(y0) + np.abs(x16.astype(np.float64)) @ np.abs(w16).T
+    W, X, Y = ctx.upload(raw), ctx.upload(x16), ctx.upload(y0)
+    ctx.gemm_xw(qtype, W, 0, X, 0, Y, 0, M, K, N, 1)
+    y = Y.download(np.float32, (N, M)).astype(np.float64)
+    assert (np.abs(y - ref) <= (K / 32 + 32) * 2.0 ** -23 * mag).all()
+    for b in (W, X, Y):
+        ctx.free(b)
+
+
 def test_gemm_accumulates_and_rejects_bad_shapes(ctx, orc):
     import zinc_amd
     M, K, N = 256, 256, 40

@@ -5,9 +5,9 @@
 // dmmv.zig:1045-1094, mul_mm_q4k.comp). X is token-major fp16 (the reference
 // keeps X column-major K x N in f32, dmmv.zig:139-155 — the same element
 // order), Y token-major f32. W stays in GGUF Q4_K / Q6_K blocks; each
-// K-step dequantises one super-block column of a 128-row tile into LDS as
+// K-step dequantises one super-block column of a row tile into LDS as
 // fp16 (value computed in f32 exactly as dequantRow, then rounded to
-// nearest even) and the four waves run v_mfma_f32_16x16x32_f16 with f32
+// nearest even) and the waves run v_mfma_f32_16x16x32_f16 with f32
 // accumulation.
 //
 // MFMA 16x16x32 f16 operand layout (lane l): A[i][k] with i = l % 16,
@@ -23,8 +23,6 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-constexpr int GT = 256;         // threads (4 waves)
-constexpr int TI = 128;         // tokens per tile
 constexpr int KS = 128;         // k per step: half a super-block
 // halfs per LDS row: 288 B (measured on the 512-token prefill: 15.45 ms
 // against 15.88 for 272 B rows, 24.6 for unpadded 256 B rows; strides that
@@ -163,22 +161,27 @@ ZH_DEV void deq_q6k_unit(const RawQ6K &r, uint32_t g, _Float16 *dst) {
 }
 
 // Tile = TI tokens x TJ weight rows, K in steps of KS = half a super-block.
-// Waves 2 x 2: wave (wi, wj) owns tokens 64 wi .. +63 and rows TJ/2 wj ..
-// +TJ/2 (4 x TJ/32 MFMA tiles). Each step the threads dequantise the tile's
+// Waves TI / 64 x 2: wave (wi, wj) owns tokens 64 wi .. +63 and rows TJ/2 wj
+// .. +TJ/2 (4 x TJ/32 MFMA tiles). Each step the threads dequantise the tile's
 // TJ x 4 units of 32 elements (UPT per thread) into LDS while the X chunks
 // of the next step and the raw weight bytes of the next two steps are in
-// flight in registers. 74 KB of
-// LDS (TJ = 128): two workgroups per CU, so one's dequantisation overlaps
-// the other's MFMAs.
-template <int QT, int TJ>
-__global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
+// flight in registers. A step's dequantisation (VALU), LDS traffic and MFMAs
+// take about a third each and hardly overlap, with one workgroup per CU (TI =
+// 256, 111 / 129 KB of LDS) as with two (TI = 128, 74 KB): what pays is less
+// of the first two per MFMA, so tiles of 256 tokens (half the dequantisation)
+// and 192 rows (1.27 x the MFMAs per LDS byte). 24576 x 4096, 512 tokens: 128
+// x 128 163 us, 256 x 128 155, 256 x 192 125 (826 TFLOP/s); 12288 rows 94 ->
+// 81; Q6_K 4096 x 12288 103 -> 91.
+template <int QT, int TJ, int TI>
+__global__ __launch_bounds__(2 * TI, 2) void k_gemm(GemmP p) {
+    constexpr int GT = 2 * TI;  // threads: TI / 64 x 2 waves
     extern __shared__ __align__(16) uint8_t lds[];
     _Float16 *xs = (_Float16 *)lds;       // [TI][LDR]
     _Float16 *ws = xs + TI * LDR;          // [TJ][LDR]
     constexpr int WJ = TJ / 2;             // weight rows per wave
     constexpr int NJ = WJ / 16, NI = 64 / 16;
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const uint32_t wi = wave & 1, wj = wave >> 1;
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const uint32_t wi = wave % (TI / 64), wj = wave / (TI / 64);
     const uint32_t n0 = blockIdx.y * TI;
     // segment of this row tile
     const uint32_t jg = blockIdx.x * TJ;
@@ -195,7 +198,7 @@ __global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
     constexpr int XC = TI * KS / 8 / GT;  // 16-byte X chunks per thread per step
-    constexpr int UPT = TJ * 4 / GT;      // units (row, 32-element group u4) per thread per step
+    constexpr int UPT = (TJ * 4 + GT - 1) / GT;  // units (row, 32-element group u4) per thread per step (the last by whole waves)
     half8 xr[XC];
     typedef typename std::conditional<QT == ZH_Q4_K, RawQ4K, RawQ6K>::type Raw;
     // the raw weight bytes (HBM) are requested two K-steps ahead, in two
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
     auto load_w = [&](uint32_t st, Raw (&wr)[UPT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < UPT; k++) {
-            const uint32_t u = k * GT + tid, r = u >> 2, u4 = u & 3;
+            const uint32_t u = k * GT + tid, r = min(u >> 2, (uint32_t)TJ - 1), u4 = u & 3;
             const uint32_t row = min(j0 + r, Ms - 1);  // rows past the segment: loaded clamped, never written
             const uint8_t *blk = Wseg + (size_t)row * p.row_bytes + (size_t)(st >> 1) * bpb;
             if constexpr (QT == ZH_Q4_K) load_q4k_unit(blk, 2 * (st & 1) + (u4 >> 1), wr[k]);
@@ -232,6 +235,7 @@ __global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
 #pragma unroll
         for (int k = 0; k < UPT; k++) {
             const uint32_t u = k * GT + tid, r = u >> 2, u4 = u & 3;
+            if (TJ * 4 % GT && k == UPT - 1 && wave >= (TJ * 4 - k * GT) / 64) break;
             // Q4_K: u4 = (sub-pair within the half, nibble) -> elements 32 u4 of the step
             if constexpr (QT == ZH_Q4_K) deq_q4k_unit(wr[k], 2 * (st & 1) + (u4 >> 1), u4 & 1, ws + r * LDR + 32 * u4);
             else deq_q6k_unit(wr[k], u4, ws + r * LDR + 32 * u4);
@@ -239,8 +243,10 @@ __global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
         __syncthreads();
         // X first: a wave's loads complete in order, so waiting for this X
         // next step does not wait for the weight bytes requested after it
-        if (st + 1 < nst) load_x(st + 1);
-        if (st + 2 < nst) load_w(st + 2, wr);
+        // (unconditional, past the end the last step again: a load behind a
+        // branch makes the compiler's wait for X drain the weight bytes too)
+        load_x(min(st + 1, nst - 1));
+        load_w(min(st + 2, nst - 1), wr);
 #pragma unroll
         for (int kk = 0; kk < KS / 32; kk++) {
             const uint32_t ko = kk * 32 + 8 * (lane / 16);
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(GT, 2) void k_gemm(GemmP p) {
         __syncthreads();
     };
     load_w(st_begin, wa);
-    if (st_begin + 1 < nst) load_w(st_begin + 1, wb);
+    load_w(min(st_begin + 1, nst - 1), wb);
     load_x(st_begin);
     for (uint32_t st = st_begin; st < nst; st += 2) {
         step(st, wa);
@@ -452,29 +458,37 @@ int zhk_gemm_multi(zh_ctx *c, uint32_t qtype, uint32_t nseg, const uint8_t *cons
     }
     for (uint32_t s = nseg; s < 3; s++) p.seg_end[s] = end;
     p.M = end;
-    const uint32_t ni = (N + TI - 1) / TI;
-    // 128-row tiles, K split when there are fewer tiles than two per CU
-    // (below); 64-row tiles only where a segment boundary needs them (every
-    // segment but the last is a whole number of tiles)
-    bool small = zh_knob("ZH_GEMM_TJ64");
-    for (uint32_t s = 0; s + 1 < nseg; s++)
-        if (M[s] % 128) small = true;
     for (uint32_t s = 0; s + 1 < nseg; s++)
         if (M[s] % 64) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "gemm: segment rows %u not a multiple of 64", M[s]);
-    const uint32_t TJv = small ? 64 : 128;
-    const uint32_t lds = (TI + TJv) * LDR * 2;
-    // Fewer tiles than two per CU (O, down, the stacked Q/K/V): split K so
-    // two workgroups share each CU (one's dequantisation overlapping the
-    // other's MFMAs), within one round of resident workgroups (rounding the
-    // split up measured slower for Q/K/V: 576 workgroups for 512 slots); at
-    // least 8 K-steps per split.
-    const uint64_t tiles = (uint64_t)((end + TJv - 1) / TJv) * ni, slots = 2ull * (uint64_t)c->cu_count;
-    p.ksplit = 1;
-    if (tiles < slots && !zh_knob("ZH_NO_SPLITK")) {
-        uint32_t sk = (uint32_t)(slots / tiles);
-        while (sk > 1 && K / KS < 8 * sk) sk--;
+    // Tile and K split by the time they should take, in K steps of a 256-token
+    // x 128-row tile (2.5 us): rounds of workgroups on the device x a
+    // workgroup's steps. Measured per step: 1.4 with 192 rows (24576 rows,
+    // 1024 tokens: 242 us in two rounds against 266 in three of 128 rows);
+    // 0.65 for a 128-token tile, 0.4 with 64 rows, in CU time (two share a
+    // CU). 96 rows cost a step as long as 128. A launch with fewer tiles than
+    // fit at once splits K within one round, at least 8 steps per split (the
+    // partial sums cost about two steps). 256 tokens from N = 129 on: 24576
+    // rows, 129 / 256 / 257 / 512 tokens 71 / 86 / 113 / 125 us against 90 /
+    // 96 / 140 / 163 in 128-token tiles; 4096 rows alike. 64-row tiles only
+    // where a segment boundary needs them.
+    const uint32_t cus = (uint32_t)c->cu_count, nst = K / KS;
+    struct { uint32_t ti, tj; float step; } const kinds[] = {{256, 192, 1.4f}, {256, 128, 1.f}, {128, 128, 0.65f}, {128, 64, 0.4f}};
+    uint32_t TI = 0, TJv = 0, ni = 0;
+    float best = 0.f;
+    for (const auto &k : kinds) {
+        bool ok = (k.ti == 128 || N > 128) && (k.tj != 192 || qtype == ZH_Q4_K);
+        for (uint32_t s = 0; s + 1 < nseg; s++) ok = ok && M[s] % k.tj == 0;
+        if (!ok || (k.tj == 64 && TI)) continue;
+        const uint32_t t = (end + k.tj - 1) / k.tj * ((N + k.ti - 1) / k.ti), slots = k.ti == 256 ? cus : 2 * cus;
+        uint32_t sk = t < slots && !zh_knob("ZH_NO_SPLITK") ? slots / t : 1;
+        while (sk > 1 && nst < 8 * sk) sk--;
+        const float time = k.step * (float)((t * sk + cus - 1) / cus) * (float)nst / (float)sk + (sk > 1 ? 2.f : 0.f);
+        if (TI && time >= best) continue;
+        TI = k.ti; TJv = k.tj; best = time;
+        ni = (N + TI - 1) / TI;
         p.ksplit = sk;
     }
+    const uint32_t lds = (TI + TJv) * LDR * 2;
     if (p.ksplit > 1) {
         void *scr = nullptr;
         int rc = zh_scratch(c, 4ull * p.ksplit * N * end, &scr);
@@ -482,9 +496,15 @@ int zhk_gemm_multi(zh_ctx *c, uint32_t qtype, uint32_t nseg, const uint8_t *cons
         p.part = (float *)scr;
     }
     dim3 grid((end + TJv - 1) / TJv, ni, p.ksplit);
-#define GL(Q, J) hipLaunchKernelGGL((k_gemm<Q, J>), grid, dim3(GT), lds, c->stream, p)
-    if (qtype == ZH_Q4_K) { if (small) GL(ZH_Q4_K, 64); else GL(ZH_Q4_K, 128); }
-    else { if (small) GL(ZH_Q6_K, 64); else GL(ZH_Q6_K, 128); }
+#define GL(Q, J, I) hipLaunchKernelGGL((k_gemm<Q, J, I>), grid, dim3(2 * I), lds, c->stream, p)
+#define GQ(Q)                                     \
+    if (TI == 256 && TJv == 128) GL(Q, 128, 256); \
+    else if (TJv == 128) GL(Q, 128, 128);         \
+    else GL(Q, 64, 128)
+    if (TJv == 192) GL(ZH_Q4_K, 192, 256);  // (Q6_K's 96 accumulators and raw bytes do not fit the registers)
+    else if (qtype == ZH_Q4_K) { GQ(ZH_Q4_K); }
+    else { GQ(ZH_Q6_K); }
+#undef GQ
 #undef GL
     if (rope && p.ksplit > 1) {
         hipLaunchKernelGGL(k_reduce_qkv_rope, dim3(N), dim3(256), 0, c->stream, p, *rope);

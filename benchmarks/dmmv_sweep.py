@@ -166,12 +166,10 @@ def measure_batched(ctx, name, qt, M, K, gate_up, ncols=(1, 2, 4, 8), iters=40):
         for i in range(2 * ncp):
             fn(i % ncp)
         ctx.sync()
-        ctx.swiglu(sep, sep, sep, 4)  # separator (kernel trace: the sweep launches no other k_swiglu)
         ctx.record(0)
         for i in range(iters):
             fn(i % ncp)
         ctx.record(1)
-        ctx.swiglu(sep, sep, sep, 4)
         ctx.sync()
         us = ctx.elapsed_ms(0, 1) * 1e3 / iters
         res["cols"][n] = {"us": round(us, 2), "us_per_col": round(us / n, 2)}

@@ -289,8 +289,9 @@ int zh_engine_generate(zh_engine *eng, const uint32_t *prompt, uint32_t n_prompt
  * ...) with base's own ctx); prompts [n_seq][n_prompt]; all sequences start
  * at start_pos; out_tokens [n_seq][max_tokens] (no EOS stop). The Q/K/V, O,
  * gate/up, down and LM-head mat-vecs run as batched DMMV launches
- * (zh_dmmv_batched), attention per sequence. Dense models whose projections
- * are Q4_K / Q6_K (ZH_ERR_UNSUPPORTED_QUANT_TYPE otherwise). */
+ * (zh_dmmv_batched), the attention of up to 16 sequences in one launch. Dense
+ * models whose projections are Q4_K / Q6_K (ZH_ERR_UNSUPPORTED_QUANT_TYPE
+ * otherwise). */
 int zh_engine_generate_batch(zh_engine *const *engines, uint32_t n_seq, const uint32_t *prompts, uint32_t n_prompt,
                              uint32_t start_pos, uint32_t max_tokens, uint32_t *out_tokens);
 /* Copy the last logits (vocab f32) to host. */

@@ -135,6 +135,7 @@ int zh_scratch(zh_ctx *c, uint64_t bytes, void **out) {
             ZH_HIP(c, hipStreamSynchronize(c->stream));
             ZH_HIP(c, hipFree(c->scratch));
             c->scratch = nullptr;
+            c->scratch_size = 0;  // (none, should the allocation below fail)
         }
         uint64_t sz = bytes < (1u << 20) ? (1u << 20) : bytes + 256;
         ZH_HIP(c, hipMalloc(&c->scratch, sz));

@@ -243,10 +243,12 @@ __global__ __launch_bounds__(2 * TI, 2) void k_gemm(GemmP p) {
         __syncthreads();
         // X first: a wave's loads complete in order, so waiting for this X
         // next step does not wait for the weight bytes requested after it
-        // (unconditional, past the end the last step again: a load behind a
-        // branch makes the compiler's wait for X drain the weight bytes too)
-        load_x(min(st + 1, nst - 1));
-        load_w(min(st + 2, nst - 1), wr);
+        // (256 tokens: unconditional, past the end the last step again, since a
+        // load behind a branch makes the compiler's wait for X drain the
+        // weight bytes too; with 128 tokens the extra loads cost a 3-layer
+        // prefill of 11 tokens 675 us against 664)
+        if (TI == 256 || st + 1 < nst) load_x(min(st + 1, nst - 1));
+        if (TI == 256 || st + 2 < nst) load_w(min(st + 2, nst - 1), wr);
 #pragma unroll
         for (int kk = 0; kk < KS / 32; kk++) {
             const uint32_t ko = kk * 32 + 8 * (lane / 16);
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(2 * TI, 2) void k_gemm(GemmP p) {
         __syncthreads();
     };
     load_w(st_begin, wa);
-    load_w(min(st_begin + 1, nst - 1), wb);
+    if (TI == 256 || st_begin + 1 < nst) load_w(min(st_begin + 1, nst - 1), wb);
     load_x(st_begin);
     for (uint32_t st = st_begin; st < nst; st += 2) {
         step(st, wa);
@@ -650,8 +652,8 @@ __global__ __launch_bounds__(256) void k_swiglu_rows_f16(const float *__restrict
 }
 
 // Causal prefill attention on the MFMA units (flash attention): workgroup =
-// one q head x AQ = 64 queries, NG groups of two waves; group g takes key
-// blocks g, g + NG, ... of AK = 64 keys, each wave 32 queries of them, and the
+// one q head x AQ = 64 queries, NG groups of waves; group g takes key
+// blocks g, g + NG, ... of AK = 64 keys, each wave 16 QT queries of them, and the
 // groups' outputs are merged at the end (log-sum-exp weights in LDS). The
 // longest query tile bounds the launch (one workgroup per CU at 512 tokens),
 // so its chain of key blocks is cut by NG. Bound by LDS traffic (1.3 us of
@@ -676,19 +678,21 @@ constexpr int AVLD = 128 + 16;   // halfs per V row: 8 rows' 32-byte pieces hit 
 constexpr uint32_t AP_GROUP = (AK * (AKLD + AVLD)) * 2;  // LDS of a group (its merge rows fit in it)
 constexpr uint32_t AP_OLD = 132;                          // floats per query of a group's output
 static_assert(AQ * AP_OLD * 4 + AQ * 8 <= AP_GROUP, "the merge rows overlay the key block");
-template <int NG>
-__global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+template <int NG, int QT>
+__global__ __launch_bounds__(NG * 256 / QT) void k_attn_prefill_mfma(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                                const uint16_t *__restrict__ vc,
                                                                const uint32_t *__restrict__ pages, uint32_t n_pages,
                                                                uint32_t cache_tokens, uint32_t nq, uint32_t nkv,
                                                                uint32_t pos0, uint32_t N, float scale,
                                                                _Float16 *__restrict__ out) {
     constexpr int HD = 128;
+    constexpr int WPG = AQ / 16 / QT, NT = 64 * WPG;  // waves and threads per group
+    constexpr int NL = AK * 16 / NT, KL = NT / 16;    // chunks per thread, keys per load
     extern __shared__ __align__(16) uint8_t lds[];
     typedef __fp16 tr4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) tr4 lds_tr4;
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const uint32_t g = wave / 2, w2 = wave % 2, tg = tid & 127, li = lane % 16, lg = lane / 16;
+    const uint32_t g = wave / WPG, w2 = wave % WPG, tg = tid % NT, li = lane % 16, lg = lane / 16;
     _Float16 *const ks = (_Float16 *)(lds + g * AP_GROUP), *const vs = ks + AK * AKLD;
     // workgroups go round robin over the XCDs: the q heads of a kv head to one
     const uint32_t G = nq / nkv, kvh = blockIdx.x % nkv, h = kvh * G + blockIdx.x / nkv;
@@ -696,10 +700,10 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
     const uint16_t *kh = kc + (size_t)kvh * cache_tokens * HD;
     const uint16_t *vh = vc + (size_t)kvh * cache_tokens * HD;
     // Q fragments (B operand): query i0 + 32 w2 + 16 t + li, d = 32 k4 + 8 lg .. +7
-    half8 qa[2][4];
+    half8 qa[QT][4];
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const float *qp = q + (size_t)min(i0 + 32 * w2 + 16 * t + li, N - 1) * nq * HD + (size_t)h * HD + 8 * lg;
+    for (int t = 0; t < QT; t++) {
+        const float *qp = q + (size_t)min(i0 + 16 * QT * w2 + 16 * t + li, N - 1) * nq * HD + (size_t)h * HD + 8 * lg;
 #pragma unroll
         for (int k4 = 0; k4 < 4; k4++) {
             const f32x4 a = *(const f32x4 *)(qp + 32 * k4), b = *(const f32x4 *)(qp + 32 * k4 + 4);
@@ -707,26 +711,28 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
                               (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
         }
     }
-    f32x4v o[2][8];  // O^T: dims 16 db + 4 lg + r of query 16 t + li
+    f32x4v o[QT][8];  // O^T: dims 16 db + 4 lg + r of query 16 t + li
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int t = 0; t < QT; t++)
 #pragma unroll
         for (int db = 0; db < 8; db++) o[t][db] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // base-2 running maxima (all lg alike), this lane's share of the sums
+    float m[QT], l[QT];  // base-2 running maxima (all lg alike), this lane's share of the sums
+#pragma unroll
+    for (int t = 0; t < QT; t++) { m[t] = -INFINITY; l[t] = 0.f; }
     const float c = scale * 1.44269504088896340736f;
     const uint32_t kmax = pos0 + min(i0 + AQ, N) - 1;  // last key any query of the workgroup sees
     const uint32_t nblk = kmax / AK + 1, nstep = (nblk + NG - 1) / NG;
-    const uint32_t q0 = pos0 + i0 + 32 * w2;
-    // the key block's K and V chunks (16 B of one key each: 8 per thread)
+    const uint32_t q0 = pos0 + i0 + 16 * QT * w2;
+    // the key block's K and V chunks (16 B of one key each: NL per thread)
     // wait in registers, requested while the previous block computes; rows
     // past kmax are loaded clamped and masked below
-    u32x4 pk[8], pv[8];
-    auto load = [&](uint32_t kb, const uint16_t *src, u32x4 (&dst)[8]) __attribute__((always_inline)) {
+    u32x4 pk[NL], pv[NL];
+    auto load = [&](uint32_t kb, const uint16_t *src, u32x4 (&dst)[NL]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < 8; it++) {  // keys 8 it + tg / 16: one page
-            const uint32_t pg = min(kb * 4 + it / 2, kmax / 16);
+        for (int it = 0; it < NL; it++) {  // keys KL it + tg / 16 (KL <= 16): one page
+            const uint32_t pg = min(kb * 4 + it * KL / 16, kmax / 16);
             uint32_t ph = pages[min(pg, n_pages - 1)] * 16;
-            const uint32_t row = 8 * (it & 1) + tg / 16, r = pg == kmax / 16 ? min(row, kmax % 16) : row;
+            const uint32_t row = it * KL % 16 + tg / 16, r = pg == kmax / 16 ? min(row, kmax % 16) : row;
             ph = ph + 16 <= cache_tokens || ph + r < cache_tokens ? ph + r : 0u;
             dst[it] = *(const u32x4 *)(src + (size_t)ph * HD + (tg % 16) * 8);
         }
@@ -740,25 +746,26 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
         const bool mine = kb < nblk;  // uniform in the group
         if (mine) {
 #pragma unroll
-            for (int it = 0; it < 8; it++) {
-                *(u32x4 *)(ks + (8 * it + tg / 16) * AKLD + (tg % 16) * 8) = pk[it];
-                *(u32x4 *)(vs + (8 * it + tg / 16) * AVLD + (tg % 16) * 8) = pv[it];
+            for (int it = 0; it < NL; it++) {
+                *(u32x4 *)(ks + (KL * it + tg / 16) * AKLD + (tg % 16) * 8) = pk[it];
+                *(u32x4 *)(vs + (KL * it + tg / 16) * AVLD + (tg % 16) * 8) = pv[it];
             }
         }
         __syncthreads();
         const bool more = kb + NG < nblk;
         if (more) load(kb + NG, kh, pk);
-        const bool sees = mine && kb * AK <= q0 + 31;  // (uniform per wave: some query of it sees the block)
-        f32x4v sc[2][4];
+        const bool sees = mine && kb * AK <= q0 + 16 * QT - 1;  // (uniform per wave: some query of it sees the block)
+        f32x4v sc[QT][4];
         if (sees) {
 #pragma unroll
             for (int jb = 0; jb < 4; jb++) {
-                sc[0][jb] = sc[1][jb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < QT; t++) sc[t][jb] = f32x4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int k4 = 0; k4 < 4; k4++) {
                     const half8 a = *(const half8 *)(ks + (16 * jb + li) * AKLD + 32 * k4 + 8 * lg);
 #pragma unroll
-                    for (int t = 0; t < 2; t++)
+                    for (int t = 0; t < QT; t++)
                         sc[t][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qa[t][k4], sc[t][jb], 0, 0, 0);
                 }
             }
@@ -766,9 +773,9 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
         if (more) load(kb + NG, vh, pv);  // (after the scores: their registers are taken until then)
         if (sees) {
             const bool whole = kb * AK + AK - 1 <= q0;  // every query sees every key
-            half8 pb[2][2];
+            half8 pb[QT][2];
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < QT; t++) {
                 const uint32_t qpos = q0 + 16 * t + li;
                 float mb = -INFINITY;
 #pragma unroll
@@ -811,18 +818,18 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
                     const half8 a = {(_Float16)t0[0], (_Float16)t0[1], (_Float16)t0[2], (_Float16)t0[3],
                                      (_Float16)t1[0], (_Float16)t1[1], (_Float16)t1[2], (_Float16)t1[3]};
 #pragma unroll
-                    for (int t = 0; t < 2; t++)
+                    for (int t = 0; t < QT; t++)
                         o[t][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb[t][s2], o[t][db], 0, 0, 0);
                 }
         }
         __syncthreads();  // the block's K / V tiles are rewritten next
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++) l[t] = xor32_sum(xor16_sum(l[t]));
+    for (int t = 0; t < QT; t++) l[t] = xor32_sum(xor16_sum(l[t]));
     if constexpr (NG == 1) {
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const uint32_t i = i0 + 32 * w2 + 16 * t + li;
+        for (int t = 0; t < QT; t++) {
+            const uint32_t i = i0 + 16 * QT * w2 + 16 * t + li;
             if (i >= N) continue;
             const float inv = 1.0f / l[t];
             _Float16 *op = out + (size_t)i * nq * HD + (size_t)h * HD + 4 * lg;
@@ -834,8 +841,8 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
     } else {
         float *const go = (float *)(lds + g * AP_GROUP), *const gm = go + AQ * AP_OLD, *const gl = gm + AQ;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const uint32_t qr = 32 * w2 + 16 * t + li;
+        for (int t = 0; t < QT; t++) {
+            const uint32_t qr = 16 * QT * w2 + 16 * t + li;
 #pragma unroll
             for (int db = 0; db < 8; db++) *(f32x4v *)(go + qr * AP_OLD + 16 * db + 4 * lg) = o[t][db];
             if (lg == 0) {
@@ -845,6 +852,7 @@ __global__ __launch_bounds__(NG * 128) void k_attn_prefill_mfma(const float *__r
         }
         __syncthreads();
         // thread: query tid / (2 NG), 64 / NG dims
+        static_assert(NT == 128, "the merge's threads per query");
         constexpr int ND = 64 / NG;
         const uint32_t mq = tid / (2 * NG), d0 = tid % (2 * NG) * ND, i = i0 + mq;
         float M = -INFINITY, w[NG], L = 0.f, r[ND];
@@ -892,12 +900,14 @@ int zhk_attn_prefill(zh_ctx *c, const float *q, const uint16_t *kc, const uint16
                      uint32_t N, float scale, _Float16 *out) {
     if (hd != 128 || nkv == 0 || nq % nkv) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "attn_prefill heads");
     const dim3 grid(nq, (N + AQ - 1) / AQ);
-    // two key blocks or fewer for any query: one group
+    // two key blocks or fewer for any query: one group, of four waves of 16
+    // queries (128 queries at 0: 8.6 us, two waves of 32 9.9, two groups 8.5;
+    // 64: 6.6 / 7.1 / 8.0)
     if (pos0 + N <= 2 * AK)
-        hipLaunchKernelGGL(k_attn_prefill_mfma<1>, grid, dim3(128), AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
+        hipLaunchKernelGGL((k_attn_prefill_mfma<1, 1>), grid, dim3(256), AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
                            cache_tokens, nq, nkv, pos0, N, scale, out);
     else
-        hipLaunchKernelGGL(k_attn_prefill_mfma<4>, grid, dim3(512), 4 * AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
+        hipLaunchKernelGGL((k_attn_prefill_mfma<4, 2>), grid, dim3(512), 4 * AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
                            cache_tokens, nq, nkv, pos0, N, scale, out);
     ZH_LAUNCH_CHECK(c);
     return ZH_OK;

@@ -267,3 +267,31 @@ def test_flash_attn_batched_edges(ctx, nh, nkv, seq_start, n, scale):
     for b in bufs:
         ctx.free(b)
 
+
+@pytest.mark.parametrize("cache_tokens", [64, 250])
+@pytest.mark.parametrize("seq_start,n", [(0, 100), (100, 60)])  # the one-group and the four-group form
+def test_flash_attn_batched_page_entries_past_the_cache(ctx, cache_tokens, seq_start, n):
+    """A token whose page entry puts it at or past cache_tokens reads cache
+    row 0, also where entry * 16 wraps or ends just below 2^32. The bound of
+    test_flash_attn_batched_matches_reference."""
+    nh, nkv = 4, 2
+    rng = np.random.default_rng(cache_tokens + seq_start)
+    pages = np.array([1, 0x0FFFFFFF, 0, cache_tokens // 16, 0xFFFFFFFF, 2, 0x1FFFFFFF, 0x10000001, 3, 0x7FFFFFFF],
+                     np.uint32)
+    k16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
+    v16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
+    q = rng.standard_normal((n, nh * 128)).astype(np.float32)
+    bufs = [ctx.upload(q), ctx.upload(k16), ctx.upload(v16), ctx.upload(pages), ctx.alloc(2 * n * nh * 128)]
+    print(f"page entries past {cache_tokens} tokens, {n} queries at {seq_start}", flush=True)
+    ctx.flash_attn_batched(*bufs[:4], len(pages), cache_tokens, bufs[4], nh, nkv, 128, seq_start, n, 0.0)
+    ctx.sync()
+    got = bufs[4].download(np.float16, n * nh * 128).astype(np.float64).reshape(n, -1)
+    t = np.arange(16 * len(pages))
+    phys = (pages.astype(np.uint64)[t // 16] * 16 + t % 16) % 2 ** 32
+    phys = np.where(phys < cache_tokens, phys, 0).astype(np.int64)
+    ref = _causal_ref(q, k16[:, phys], v16[:, phys], np.arange(len(pages)), nh, nkv, seq_start, 1 / np.sqrt(128))
+    bound = 4e-3 * np.abs(ref).reshape(n, nh, 128).max(axis=2).repeat(128, axis=1) + 1e-3
+    err = np.abs(got - ref)
+    assert (err <= bound).all(), (err.max(), np.unravel_index(err.argmax(), err.shape))
+    for b in bufs:
+        ctx.free(b)

@@ -731,9 +731,12 @@ __global__ __launch_bounds__(NG * 256 / QT) void k_attn_prefill_mfma(const float
 #pragma unroll
         for (int it = 0; it < NL; it++) {  // keys KL it + tg / 16 (KL <= 16): one page
             const uint32_t pg = min(kb * 4 + it * KL / 16, kmax / 16);
-            uint32_t ph = pages[min(pg, n_pages - 1)] * 16;
+            const uint32_t page = pages[min(pg, n_pages - 1)];
             const uint32_t row = it * KL % 16 + tg / 16, r = pg == kmax / 16 ? min(row, kmax % 16) : row;
-            ph = ph + 16 <= cache_tokens || ph + r < cache_tokens ? ph + r : 0u;
+            // (an entry past the cache reads row 0; the entry is compared, not
+            // its token, which an entry from 2^28 on wraps)
+            uint32_t ph = page * 16 + r;
+            ph = page < cache_tokens / 16 || ph < cache_tokens ? ph : 0u;
             dst[it] = *(const u32x4 *)(src + (size_t)ph * HD + (tg % 16) * 8);
         }
     };

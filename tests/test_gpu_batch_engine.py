@@ -93,6 +93,42 @@ def test_batch_attention_edges(ctx, n_seq, prefill, heads, paged):
     base.deinit()
 
 
+@pytest.mark.parametrize("heads", [2, 8, 16])  # 1, 4 and 8 per kv head
+def test_batch_attention_q_past_f16(ctx, heads):
+    """Query norm weights of 2^15 put q's components far past f16's 65504:
+    tokens and logits as alone on the attention kernel that multiplies in
+    f32."""
+    import ctypes as C
+    import zinc_amd
+    from zinc_amd.hip import lib
+    print(f"batch attention, q past f16, heads {heads}", flush=True)
+    cfg = dict(CFG, n_layers=2, n_heads=heads, vocab=1024)
+    base = zinc_amd.InferenceEngine(ctx, cfg)
+    w = np.full(128, 2.0 ** 15, np.float32)
+    for layer in range(2):
+        b, off, n = C.c_void_p(), C.c_uint64(), C.c_uint64()
+        ctx.check(lib().zh_engine_tensor(base.h, (layer + 1) << 8 | 6, C.byref(b), C.byref(off), C.byref(n)))
+        assert n.value == w.nbytes
+        ctx.check(lib().zh_buf_upload(ctx.h, b, off.value, C.c_void_p(w.ctypes.data), w.nbytes))
+    engines = [base] + [base.share(ctx) for _ in range(2)]
+    prompts = np.array([[5], [600], [71]], np.uint32)
+    solo, logits = [], []
+    for v, e in enumerate(engines):
+        e.set_fused_attn(False)
+        e.prefill_kv_random(200, 400 + v)
+        solo.append(e.generate(prompts[v].tolist(), 4, start_pos=200))
+        logits.append(e.logits())
+        e.prefill_kv_random(200, 400 + v)
+    assert zinc_amd.InferenceEngine.generate_batch(engines, prompts, 4, start_pos=200) == solo
+    for v, e in enumerate(engines):
+        lg = e.logits()
+        assert np.isfinite(lg).all()
+        assert np.allclose(lg, logits[v], rtol=1e-3, atol=1e-4 + 1e-3 * np.abs(logits[v]).max()), v
+    for e in engines[1:]:
+        e.deinit()
+    base.deinit()
+
+
 def test_batch_rejects_foreign_engines(ctx):
     import zinc_amd
     a = zinc_amd.InferenceEngine(ctx, dict(CFG, n_layers=2))

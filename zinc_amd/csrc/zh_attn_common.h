@@ -299,8 +299,8 @@ template <int G> constexpr int ar_waves() { return 8; }
 // [q_norm | k_norm], [RoPE row | -]; then the new K / V row as f16 (512 B)
 template <int G> constexpr uint32_t ar_qc() { return (G * FD_HD * 4 + 1023) / 1024; }
 template <int G> constexpr uint32_t ar_small() { return (ar_qc<G>() + 3) * 1024 + 512; }
-// q's MFMA fragments (8 steps x 64 lanes x (hi, lo) 8 bytes) and the
-// heads' 1 / rms
+// q's MFMA fragments (8 steps x 64 lanes x (hi, lo) 8 bytes; or 8 steps x 4
+// x G heads x 3 pieces) and the heads' 1 / rms (then their scales)
 constexpr uint32_t AR_QFRAG = 8 * 64 * 16 + 64 * 4;
 template <int G, int AW = ar_waves<G>()>
 constexpr uint32_t ar_lds_bytes() {
@@ -366,12 +366,42 @@ ZH_DEV uint32_t attn_ring_prefetch(const AttnP &p, uint32_t kvh, uint32_t c, uin
     return n;
 }
 
+// x = sum of N f16 pieces, each the rounded rest of those before it, for 4
+// values (piece k of value j in h[k][j])
+template <int N>
+ZH_DEV void split_f16(const float (&x)[4], half4 (&h)[N]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float r = x[j];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            h[k][j] = (_Float16)r;
+            r -= (float)h[k][j];  // exact
+        }
+    }
+}
+// NP = 3: q is scaled by a power of two that puts the head's largest
+// component at 2^13 to 2^14 before the rotation (which grows it by at most
+// sqrt 2), p by 2^14: three pieces then hold an f32 exactly, less at most
+// 2^-25 of those scaled units, and no q overflows f16. For the batched launch,
+// whose predecessor multiplied in f32. Distance from 64 bits (2-norm, 2 to 4
+// sequences, 32 / 8 heads, f32 kernel / three pieces / two): 4096 tokens 2.1 / 2.0 / 2.8e-7,
+// scores four times as wide 4.9 / 4.8 / 8.4e-7; 16000 tokens 2.4 / 2.1 / 3.2e-7. Eight sequences of 8 layers
+// at 4096 tokens 870 us a step with three pieces, 857 with two.
+constexpr float AR_PSCALE = 16384.f;
+// the exponent field of that power for a head whose largest component is amax
+ZH_DEV uint32_t ar_qscale_field(float amax) {
+    const uint32_t e = __float_as_uint(amax) >> 23;  // (amax >= 0)
+    return e == 255u ? 127u : min(267u - e, 253u);
+}
+
 // AW waves (4 or 8: one or two groups of four taking alternate sub-chunks);
 // COH: q and the new token's k / v were written by other workgroups of the
 // same launch (read at system scope), and the merged output is read by other
 // workgroups of it (stored at device scope). pre: sub-chunks 0 .. pre-1
-// already copied (attn_ring_prefetch, page entries included).
-template <int G, bool FUSED, int AW, bool COH>
+// already copied (attn_ring_prefetch, page entries included). NP: f16 pieces
+// of q and of the probabilities, 2 (22 bits) or 3 (the f32 values, FUSED only).
+template <int G, bool FUSED, int AW, bool COH, int NP = 2>
 ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *lds, uint32_t pre = 0) {
     constexpr int AT = AW * 64, NG = AW / 4;  // threads, groups
     constexpr uint32_t QC = ar_qc<G>();
@@ -437,9 +467,11 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
     // 16-dim steps s, RMS-normalised and roped in place (the RoPE partner of
     // dim d < 64, d + 64, is step s + 4 of the same lane), then split into
     // f16 hi + lo parts so that the f16 products carry the f32 q exactly
-    // enough (|q - hi - lo| <= 2^-22 |q|).
+    // enough (|q - hi - lo| <= 2^-22 |q|), or scaled and split in three.
+    static_assert(NP == 2 || FUSED, "three pieces: q is scaled where it is normalised");
     const uint32_t fg = lane & 15, fq = lane >> 4;
-    half4 qh[8], ql[8];
+    half4 qf[8][NP];
+    float score_scale = p.scale;  // of this lane's head fg
     {
         // computed once per workgroup and shared through LDS: the heads' RMS
         // (wave g: head g), then group 0's wave w the dims of steps w and
@@ -451,7 +483,13 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
                 const float *qs = (const float *)sm + g * FD_HD;
                 const float a = qs[lane], b = qs[lane + 64];
                 const float sq = wave_sum(fmaf(a, a, b * b));
-                if (lane == 0) rinv[g] = 1.0f / sqrtf(sq / (float)FD_HD + p.eps);
+                const float ri = 1.0f / sqrtf(sq / (float)FD_HD + p.eps);
+                if (lane == 0) rinv[g] = ri;
+                if (NP == 3) {
+                    const float *qw = (const float *)(sm + (QC + 1) * 1024);
+                    const float m = wave_max(fmaxf(fabsf(qw[lane] * (a * ri)), fabsf(qw[lane + 64] * (b * ri))));
+                    if (lane == 0) ((uint32_t *)rinv)[FD_MAXG + g] = ar_qscale_field(m);
+                }
             }
             lds_bar();
         }
@@ -474,26 +512,45 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
                     hi[j] = a * sn + b * co;
                 }
             }
-            half4 h0, l0, h1, l1;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const float x = fg < (uint32_t)G ? lo[j] : 0.f, y = fg < (uint32_t)G ? hi[j] : 0.f;
-                h0[j] = (_Float16)x;
-                l0[j] = (_Float16)(x - (float)h0[j]);
-                h1[j] = (_Float16)y;
-                l1[j] = (_Float16)(y - (float)h1[j]);
+                lo[j] = fg < (uint32_t)G ? lo[j] : 0.f;
+                hi[j] = fg < (uint32_t)G ? hi[j] : 0.f;
             }
-            *(half4 *)(frag + (pi * 64 + lane) * 16) = h0;
-            *(half4 *)(frag + (pi * 64 + lane) * 16 + 8) = l0;
-            *(half4 *)(frag + ((pi + 4) * 64 + lane) * 16) = h1;
-            *(half4 *)(frag + ((pi + 4) * 64 + lane) * 16 + 8) = l1;
+            if constexpr (NP == 2) {
+                half4 h0[2], h1[2];
+                split_f16(lo, h0);
+                split_f16(hi, h1);
+                *(half4 *)(frag + (pi * 64 + lane) * 16) = h0[0];
+                *(half4 *)(frag + (pi * 64 + lane) * 16 + 8) = h0[1];
+                *(half4 *)(frag + ((pi + 4) * 64 + lane) * 16) = h1[0];
+                *(half4 *)(frag + ((pi + 4) * 64 + lane) * 16 + 8) = h1[1];
+            } else if (fg < (uint32_t)G) {
+                const float qs = __uint_as_float(((const uint32_t *)rinv)[FD_MAXG + fg] << 23);
+#pragma unroll
+                for (int j = 0; j < 4; j++) { lo[j] *= qs; hi[j] *= qs; }
+                half4 h0[NP], h1[NP];
+                split_f16(lo, h0);
+                split_f16(hi, h1);
+#pragma unroll
+                for (int k = 0; k < NP; k++) {
+                    *(half4 *)(frag + (((pi * 4 + fq) * G + fg) * NP + k) * 8) = h0[k];
+                    *(half4 *)(frag + ((((pi + 4) * 4 + fq) * G + fg) * NP + k) * 8) = h1[k];
+                }
+            }
         }
         lds_bar();
+        // (three pieces: the G heads only, in the space of 16 rows of two; the
+        // lanes past them repeat the last head, whose probabilities are zeroed)
+        const uint32_t gl = min(fg, (uint32_t)G - 1);
+        if constexpr (NP == 3)  // (a power of two: the product is exact)
+            score_scale *= __uint_as_float((254u - ((const uint32_t *)rinv)[FD_MAXG + gl]) << 23);
 #pragma unroll
-        for (int s8 = 0; s8 < 8; s8++) {
-            qh[s8] = *(const half4 *)(frag + (s8 * 64 + lane) * 16);
-            ql[s8] = *(const half4 *)(frag + (s8 * 64 + lane) * 16 + 8);
-        }
+        for (int s8 = 0; s8 < 8; s8++)
+#pragma unroll
+            for (int k = 0; k < NP; k++)
+                qf[s8][k] = *(const half4 *)(frag + (NP == 2 ? (s8 * 64 + lane) * 16 + k * 8
+                                                             : (((s8 * 4 + fq) * G + gl) * NP + k) * 8));
     }
     TRACE_OPS(9);
     // ---- the new token's k / v (the owner only)
@@ -601,14 +658,31 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
             }
             // scores
             floatx4 d1 = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (NP == 2) {
 #pragma unroll
-            for (int s8 = 0; s8 < 8; s8++) {
-                d1 = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], qh[s8], d1, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], ql[s8], d1, 0, 0, 0);
+                for (int s8 = 0; s8 < 8; s8++) {
+                    d1 = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], qf[s8][0], d1, 0, 0, 0);
+                    d1 = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], qf[s8][1], d1, 0, 0, 0);
+                }
+            } else {
+                // each step's first pieces by themselves and summed pairwise,
+                // the small pieces in a chain of their own: an MFMA drops low
+                // bits of the smaller of its summands, and as one chain the
+                // result was up to 1.5 times as far from 64 bits
+                floatx4 d2 = {0.f, 0.f, 0.f, 0.f}, e[8];
+#pragma unroll
+                for (int k = NP - 1; k > 0; k--)
+#pragma unroll
+                    for (int s8 = 0; s8 < 8; s8++)
+                        d2 = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], qf[s8][k], d2, 0, 0, 0);
+#pragma unroll
+                for (int s8 = 0; s8 < 8; s8++)
+                    e[s8] = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[s8], qf[s8][0], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                d1 = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7])) + d2;
             }
             float sc[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++) sc[r] = ts + tb + 4 * fq + r < t1 ? d1[r] * p.scale : -INFINITY;  // dot * scale
+            for (int r = 0; r < 4; r++) sc[r] = ts + tb + 4 * fq + r < t1 ? d1[r] * score_scale : -INFINITY;  // dot * scale
             float m = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
             m = xor16_max(m);
             m = xor32_max(m);
@@ -625,13 +699,11 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
             lsum = xor32_sum(lsum);
             l_run = fmaf(l_run, f, lsum);
             m_run = mn;
-            half4 ph, pl;
+            half4 pf[NP];
+            if constexpr (NP == 3)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const _Float16 h = (_Float16)pr[r];
-                ph[r] = h;
-                pl[r] = (_Float16)(pr[r] - (float)h);
-            }
+                for (int r = 0; r < 4; r++) pr[r] *= AR_PSCALE;
+            split_f16(pr, pf);
             // rescale the output rows (heads 4 fq + r) by their heads' factors
             // (lane h, fq = 0, holds head h's)
             float fr[4];
@@ -639,10 +711,19 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
             for (int r = 0; r < 4; r++) fr[r] = G > 4 && fq ? lane_f(f, 4 + r) : lane_f(f, r);
 #pragma unroll
             for (int n = 0; n < 8; n++) {
+                if constexpr (NP == 2) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[n][r] *= fr[r];
-                acc[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vf[n], acc[n], 0, 0, 0);
-                acc[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vf[n], acc[n], 0, 0, 0);
+                    for (int r = 0; r < 4; r++) acc[n][r] *= fr[r];
+                    acc[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(pf[0], vf[n], acc[n], 0, 0, 0);
+                    acc[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(pf[1], vf[n], acc[n], 0, 0, 0);
+                } else {  // (likewise)
+                    floatx4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int k = NP - 1; k > 0; k--) t = __builtin_amdgcn_mfma_f32_16x16x16f16(pf[k], vf[n], t, 0, 0, 0);
+                    t += __builtin_amdgcn_mfma_f32_16x16x16f16(pf[0], vf[n], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[n][r] = fmaf(acc[n][r], fr[r], t[r]);
+                }
             }
         }
         if (k < 2) TRACE_OPS(6 + 2 * k);
@@ -665,6 +746,9 @@ ZH_DEV void attn_ring_body(const AttnP &p, uint32_t kvh, uint32_t c, uint8_t *ld
         const uint32_t g = 4 * fq + r;
         if (g < (uint32_t)G) {
             f32x4 *o = (f32x4 *)(wo + (wave * G + g) * FD_HD + 8 * fg);
+            if constexpr (NP == 3)
+#pragma unroll
+                for (int n = 0; n < 8; n++) acc[n][r] *= 1.f / AR_PSCALE;
             o[0] = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
             o[1] = f32x4{acc[4][r], acc[5][r], acc[6][r], acc[7][r]};
         }

@@ -121,14 +121,17 @@ int zh_dmmv_supported(uint32_t qtype, uint32_t K);
  * dmmv_q6k_batch.comp). X: f32 [num_cols][K] (column v at X + v*K*4 bytes,
  * 16-byte aligned offset); Y: f32 [num_cols][M] (= or += when acc_mode == 1).
  * qtype Q4_K or Q6_K, K % 256 == 0, num_cols 1..ZH_DMMV_MAX_COLS. The weights
- * stream from HBM once for all columns. */
+ * stream from HBM once for all columns (13 to 16 columns of Q6_K: twice; K
+ * past 16384, and two columns of a small Q6_K matrix of K % 2048 != 0: once
+ * per column). */
 #define ZH_DMMV_MAX_COLS 16
 int zh_dmmv_batched(zh_ctx *ctx, uint32_t qtype, const zh_buf *W, uint64_t a_off, const zh_buf *X, uint64_t x_off,
                     zh_buf *Y, uint64_t y_off, uint32_t M, uint32_t K, uint32_t num_cols, uint32_t acc_mode);
-/* (The columns agree with zh_dmmv run per column to the f32 summation
- * floor; bit for bit where zh_dmmv runs the same tile kernels, i.e. not for
- * Q4_K at K = 2048 / 4096, which zh_dmmv streams with another summation
- * order.) */
+/* (A column does not depend on the other columns of the call. It equals
+ * zh_dmmv of that column bit for bit, except where zh_dmmv runs a kernel with
+ * another summation order: Q4_K at K = 2048 and 4096, odd row counts, Q6_K at
+ * K = 14336 and 16384 and Q6_K of 65536 rows or more. There the two agree to
+ * the f32 summation floor, and a call of one column may run zh_dmmv's kernel.) */
 /* Y[v] = silu(Wg X[v]) * (Wu X[v]) for v < num_cols (Q4_K), the batched form of
  * zh_dmmv_fused_gate_up_swiglu below; layouts as zh_dmmv_batched. */
 int zh_dmmv_fused_gate_up_swiglu_batched(zh_ctx *ctx, uint32_t qtype, const zh_buf *Wg, uint64_t g_off,

@@ -2,15 +2,16 @@
 skinny GEMM of recordBatchDispatchPush, dmmv.zig:880-925) through the C ABI.
 
 Every column of a batched launch must equal the one-vector DMMV of that
-column bit for bit where the one-vector path runs the tile kernels (the
-weight tile is shared, the per-column arithmetic is the one-vector
-kernel's); Q4_K with K = 2048 / 4096 runs the streaming kernel one vector at
-a time, whose half-super-block partial sums round in another order, so there
-the columns agree to the f32 summation floor (2^-20 of sum |w x|). Every
-column meets the oracle bar of the one-vector kernels: |gpu - ref| <= 1e-4 +
-1e-3 |ref| (+ the f32 dot-product noise floor of
-test_gpu_kernels.assert_dot_close). Column counts cover the 4-, 2- and
-1-vector launches and their mixtures (3, 5 and 8 columns)."""
+column bit for bit (the weights are shared, the per-column arithmetic is the
+one-vector kernel's), except where the one-vector path sums in another order:
+Q4_K with K = 2048 / 4096 (the streaming kernel's half-super-block partial
+sums), odd row counts (the team kernel), Q6_K at 56 and 64 super-blocks and
+the LM head's height (the lane-per-block kernel). There the columns agree to
+the f32 summation floor (2^-20 of sum |w x|). Every column meets the oracle
+bar of the one-vector kernels: |gpu - ref| <= 1e-4 + 1e-3 |ref| (+ the f32
+dot-product noise floor of test_gpu_kernels.assert_dot_close). Column counts
+cover the matrix-unit launches of 1 to 4 groups of 4 vectors (Q6_K past 12 in
+two), the tile launches of 2 and 4 and the one-vector launch."""
 import numpy as np
 import pytest
 
@@ -82,20 +83,23 @@ def test_batched_equals_single_columns(ctx, orc, qt, M, K, ncol):
 @pytest.mark.parametrize("qt", [12, 14])
 @pytest.mark.parametrize("M,nb,ncol", [(1, 1, 2), (15, 2, 4), (17, 3, 16), (129, 2, 5), (70, 5, 9), (33, 9, 12),
                                        (300, 15, 13), (4100, 17, 2), (50, 33, 16), (31, 49, 8), (16, 64, 3),
-                                       (40, 65, 2)])
+                                       (40, 65, 2),
+                                       # every width class and group count with an even row count
+                                       (2, 1, 3), (16, 2, 2), (18, 3, 12), (130, 5, 16), (34, 9, 12), (30, 31, 9),
+                                       (32, 49, 8), (46, 63, 5), (48, 8, 9), (30, 16, 12), (34, 24, 13), (50, 48, 16)])
 def test_batched_edges_equal_single_columns(ctx, orc, qt, M, nb, ncol):
     """Row counts off the 16-row tiles, K of 1 to 65 super-blocks (partial
     slabs of 16; past 64 one vector at a time), rows that start 2-byte aligned
     (odd Q6_K widths), every group count of 4 vectors: each column equals its
     one-vector DMMV (to the summation floor where that runs the streaming
-    kernel, or the lane-per-block kernel of Q6_K widths off 8 super-blocks
-    or past 48, which sum in another order)."""
+    kernel, the team kernel of odd row counts, or the lane-per-block kernel
+    of Q6_K at 56 and 64 super-blocks, which sum in another order)."""
     K = 256 * nb
     print(f"batched edges q{qt} {M}x{K} cols {ncol}", flush=True)
     W = orc.synth_tensor(qt | 0x100 if qt == 12 else qt, M, K, 91 + ncol, 1)
     X = np.stack([orc.synth_normal_f32(K, 92, 10 + v) for v in range(ncol)])
     Wb, Xb, Yb = ctx.upload(W), ctx.upload(X), ctx.alloc(4 * M * ncol)
-    loose = _ring(qt, K) or (qt == 14 and (nb % 8 != 0 or nb > 48)) or nb > 64 or M % 2 == 1  # (odd rows: the team kernel)
+    loose = _ring(qt, K) or (qt == 14 and nb in (56, 64)) or M % 2 == 1
     ctx.dmmv_batched(qt, Wb, 0, Xb, 0, Yb, 0, M, K, ncol)
     Y = Yb.download(np.float32, M * ncol).reshape(ncol, M)
     for v in range(ncol):

@@ -436,8 +436,10 @@ static bool tile_pays(uint32_t nv, uint32_t rows, uint32_t K) {
 // vectors on the matrix units (zh_dmmv_mfma.hip), or 2 or 4 on the tile
 // kernels where those are faster; a single vector, and shapes outside both,
 // one vector at a time. Per vector the arithmetic is that of the one-vector
-// tile kernel on every path, so every output equals its single-vector DMMV
-// bit for bit.
+// tile kernel, so an output does not depend on the other vectors and equals
+// the single-vector zhk_dmmv_lpb bit for bit, except where that streams (Q4_K
+// at K = 2048 / 4096) or sums in the lane-per-block kernel's order (Q6_K at 56
+// and 64 super-blocks and from 65536 rows on).
 int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const uint8_t *const *W, const uint8_t *W2,
                      const uint32_t *M, uint32_t K, uint32_t n_vec, const float *const *x, const void *const *xq,
                      float *const *y, const float *norm_w, float eps, uint32_t acc) {
@@ -476,7 +478,8 @@ int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const u
                 continue;
             }
         }
-        // (two vectors of a small Q6_K matrix off the tile kernels: one by one, 7.6 us against 9.0)
+        // (two vectors of a small Q6_K matrix off the tile kernels: one by one,
+        // 512 x 512 7.6 us against 9.0)
         if (mfma && left > 1 && !(left == 2 && tile_pays(2, rows, K))) {
             const int rc = zhk_dmmv_mfma(c, qtype, mode, nseg, W, W2, M, K, left, x ? x + v0 : nullptr,
                                          x ? nullptr : xq + v0, y + v0, n_vec, norm_w, eps, acc);

@@ -151,7 +151,9 @@ __global__ __launch_bounds__(LPB_T, ZH_LPB_MINB) void k_dmmv_q4k_lpb(LpbP p) {
 // budget, so a lane owns half a super-block (128 elements, h = half index):
 // ql[64h..64h+64), qh[32h..32h+32), sc[8h..8h+8), d.
 // ---------------------------------------------------------------------------
-template <int TL, int R>
+// TREE: the halves are summed pairwise from neighbours up, as the tile kernels
+// and the batched launch (k_bmm) sum them (else from the two ends of the team).
+template <int TL, int R, bool TREE>
 __global__ __launch_bounds__(LPB_T, ZH_LPB_MINB) void k_dmmv_q6k_lpb(LpbP p) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     __shared__ float red[4];
@@ -254,7 +256,8 @@ __global__ __launch_bounds__(LPB_T, ZH_LPB_MINB) void k_dmmv_q6k_lpb(LpbP p) {
         }
         constexpr int TLW = TL > 64 ? 64 : TL;
         constexpr int STRIDE = TLW / R;
-        float res = team_reduce_multi<TLW, R>(part, tlane % TLW);
+        static_assert(!TREE || R == 1, "one row per team");
+        float res = TREE ? team_sum_dpp<TLW>(part[0]) : team_reduce_multi<TLW, R>(part, tlane % TLW);
         const int idx = owner_index<TLW, R>(tlane % TLW);
         if (TL > 64) {
             __shared__ float xred[4][R];
@@ -572,7 +575,18 @@ static int launch_q4k(zh_ctx *c, const LpbP &p, uint32_t wgs, uint32_t lds) {
 }
 template <int TL>
 static int launch_q6k(zh_ctx *c, const LpbP &p, uint32_t wgs, uint32_t lds) {
-    hipLaunchKernelGGL((k_dmmv_q6k_lpb<TL, 1>), dim3(wgs), dim3(LPB_T), lds, c->stream, p);
+    // Rows of no multiple of 2048 elements, up to 64 super-blocks: the batched
+    // launch's summation order, so that a column of a batch equals its
+    // one-vector result at these widths too (at the others this kernel is the
+    // exception the batched entry points state).
+    const uint32_t nb = p.K / 256;
+    if constexpr (TL <= 128)
+        if (nb % 8) {
+            hipLaunchKernelGGL((k_dmmv_q6k_lpb<TL, 1, true>), dim3(wgs), dim3(LPB_T), lds, c->stream, p);
+            ZH_LAUNCH_CHECK(c);
+            return ZH_OK;
+        }
+    hipLaunchKernelGGL((k_dmmv_q6k_lpb<TL, 1, false>), dim3(wgs), dim3(LPB_T), lds, c->stream, p);
     ZH_LAUNCH_CHECK(c);
     return ZH_OK;
 }

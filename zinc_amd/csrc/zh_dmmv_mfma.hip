@@ -11,7 +11,8 @@
 // combination, the block scales and the f32 accumulation are lane-local and
 // run in the one-vector tile kernels' order (zh_dmmv_lpb.hip): super-blocks
 // (Q6_K: their halves) one by one, then summed pairwise in an aligned binary
-// tree. Every output therefore equals its one-vector DMMV bit for bit.
+// tree. Every output therefore equals its one-vector DMMV on those kernels bit
+// for bit (and on k_dmmv_q6k_lpb at widths of no multiple of 2048).
 #include "zh_device.h"
 #include "zh_internal.h"
 

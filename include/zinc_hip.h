@@ -123,7 +123,9 @@ int zh_dmmv_supported(uint32_t qtype, uint32_t K);
  * qtype Q4_K or Q6_K, K % 256 == 0, num_cols 1..ZH_DMMV_MAX_COLS. The weights
  * stream from HBM once for all columns (13 to 16 columns of Q6_K: twice; K
  * past 16384, and two columns of a small Q6_K matrix of K % 2048 != 0: once
- * per column). */
+ * per column). Allocates nothing: the quantised columns lie in a 1 MiB block
+ * that the context holds, so a call recorded in a graph must not be replayed
+ * beside another batched call of its context. */
 #define ZH_DMMV_MAX_COLS 16
 int zh_dmmv_batched(zh_ctx *ctx, uint32_t qtype, const zh_buf *W, uint64_t a_off, const zh_buf *X, uint64_t x_off,
                     zh_buf *Y, uint64_t y_off, uint32_t M, uint32_t K, uint32_t num_cols, uint32_t acc_mode);

@@ -172,3 +172,29 @@ def test_batched_rejects_bad_arguments(ctx):
     assert e.value.name == "InvalidArgument"
     for b in (W, X, Y):
         ctx.free(b)
+
+
+def test_batched_allocates_nothing():
+    """The first batched calls of 16 contexts leave the device's free memory
+    as it is (the operands have a place from the context's creation on, also
+    the largest: 16 columns of K = 16384)."""
+    import torch
+    import zinc_amd
+    M, K, ncol = 256, 16384, 16
+    print("batched dmmv allocations", flush=True)
+    ctxs = [zinc_amd.Context(0) for _ in range(16)]
+    W, X, Y = ctxs[0].alloc(M * K // 256 * 144), ctxs[0].alloc(4 * K * ncol), ctxs[0].alloc(4 * M * ncol)
+    for c in ctxs:  # each stream has run: the same kernel file's one-vector route, which needs no operands
+        c.dmmv_batched(12, W, 0, X, 0, Y, 0, M, K, 1)
+        c.sync()
+    ctxs[0].dmmv_batched(12, W, 0, X, 0, Y, 0, M, K, ncol)  # (its code is loaded)
+    ctxs[0].sync()
+    free = torch.cuda.mem_get_info()[0]
+    for c in ctxs[1:]:
+        c.dmmv_batched(12, W, 0, X, 0, Y, 0, M, K, ncol)
+        c.sync()
+    assert free - torch.cuda.mem_get_info()[0] < 4 << 20  # (the runtime's page granularity is 2 MiB)
+    for b in (W, X, Y):
+        ctxs[0].free(b)
+    for c in ctxs:
+        c.close()

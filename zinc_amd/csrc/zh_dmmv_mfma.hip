@@ -39,6 +39,12 @@ constexpr uint32_t bm_image_bytes(uint32_t K, uint32_t G) { return K / 64 * G * 
 // float4s of scales per 256 elements and vector: Q4_K one per 64 elements
 // (xs, sum of x; twice), Q6_K one per 32 (xs, -32 x the two 16-element sums)
 constexpr uint32_t bm_scales(uint32_t qtype) { return qtype == ZH_Q4_K ? 4u : 8u; }
+constexpr uint32_t bm_scale_bytes(uint32_t qtype, uint32_t K, uint32_t G) { return K / 256 * bm_scales(qtype) * 4 * G * 16; }
+// (the widest K and most groups of zhk_dmmv_mfma)
+constexpr uint32_t BM_MAXK = 4 * BM_SLAB * 256;
+static_assert(bm_image_bytes(BM_MAXK, 4) + bm_scale_bytes(ZH_Q4_K, BM_MAXK, 4) + 3 * BM_MAXV * 8 <= ZH_BMM_WS &&
+                  bm_image_bytes(BM_MAXK, 3) + bm_scale_bytes(ZH_Q6_K, BM_MAXK, 3) + 3 * BM_MAXV * 8 <= ZH_BMM_WS,
+              "the context's workspace");
 
 struct BmStageP {
     const float *x[BM_MAXV];    // f32 vectors, or
@@ -542,7 +548,7 @@ static int bm_launch_g(zh_ctx *c, BmP &p, uint32_t G) {
 bool zhk_dmmv_mfma_fits(uint32_t qtype, int mode, uint32_t nseg, const uint8_t *const *W, const uint8_t *W2,
                         const uint32_t *M, uint32_t K) {
     const uint32_t nb = K / 256, unit_rows = nb > 8 ? 16 : nb > 4 ? 32 : nb > 2 ? 64 : 128;
-    bool fits = K % 256 == 0 && nb && nb <= 4 * BM_SLAB && nseg >= 1 && nseg <= 3 &&
+    bool fits = K % 256 == 0 && nb && K <= BM_MAXK && nseg >= 1 && nseg <= 3 &&
                 (qtype == ZH_Q4_K || qtype == ZH_Q6_K) &&
                 (mode == LPB_PLAIN || (qtype == ZH_Q4_K && nseg == 1 && ((uintptr_t)W2 & 15) == 0));
     // 16-byte aligned matrices; stacked ones at least a unit tall
@@ -565,10 +571,7 @@ int zhk_dmmv_mfma(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const uint
         const uint32_t nv = left <= most ? left : qtype == ZH_Q6_K ? 8u : 16u;
         // waves that split K: all from 9 super-blocks on
         const uint32_t G = (nv + 3) / 4, NW = bm_waves(qtype, G), unit_rows = nb > 8 ? 16 : nb > 4 ? 32 : nb > 2 ? 64 : 128;
-        const uint32_t img = bm_image_bytes(K, G), scb = nb * bm_scales(qtype) * 4 * G * 16;
-        void *scr = nullptr;
-        const int rc = zh_scratch(c, img + scb + 3 * BM_MAXV * sizeof(float *), &scr);
-        if (rc) return rc;
+        const uint32_t img = bm_image_bytes(K, G), scb = bm_scale_bytes(qtype, K, G);
         BmStageP sp = {};
         BmP p = {};
         for (uint32_t v = 0; v < nv; v++) {
@@ -577,9 +580,9 @@ int zhk_dmmv_mfma(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const uint
             for (uint32_t s = 0; s < nseg; s++) sp.y[s][v] = y[s * y_stride + v0 + v];
         }
         sp.norm_w = x ? norm_w : nullptr; sp.eps = eps; sp.K = K; sp.G = G; sp.q6 = qtype == ZH_Q6_K;
-        sp.img = (uint8_t *)scr;
-        sp.sc = (float4 *)((uint8_t *)scr + img);
-        sp.ytab = (float **)((uint8_t *)scr + img + scb);
+        sp.img = (uint8_t *)c->bmm_ws;
+        sp.sc = (float4 *)(sp.img + img);
+        sp.ytab = (float **)(sp.img + img + scb);
         hipLaunchKernelGGL(k_bmm_stage, dim3(nv, (K + 1023) / 1024), dim3(256), 0, c->stream, sp);
         ZH_LAUNCH_CHECK(c);
         uint32_t end = 0;

@@ -42,6 +42,11 @@ struct zh_ctx {
     // Stream-ordered scratch for zh_dmmv's activation quantisation.
     void *scratch = nullptr;
     uint64_t scratch_size = 0;
+    // ZH_BMM_WS bytes: the activation operands of zhk_dmmv_mfma's current
+    // launch. Held from zh_init to zh_destroy, so that a batched DMMV neither
+    // allocates nor leaves a recorded launch pointing at freed memory, as the
+    // growing scratch would.
+    void *bmm_ws = nullptr;
     // Other contexts run kernels on this device at the same time (engines
     // sharing weights): kernels must not wait on workgroups of their own grid
     // that may not be resident (the attention merge then needs no waiting).
@@ -100,6 +105,8 @@ static inline uint64_t zh_tensor_bytes(uint32_t t, uint64_t rows, uint64_t cols)
     return rows * (cols / zh_block_size(t)) * zh_bytes_per_block(t);
 }
 static inline uint64_t zh_xq_bytes_int(uint32_t K) { return (uint64_t)(K / 32) * 108; }
+
+constexpr uint64_t ZH_BMM_WS = 1u << 20;
 
 // ---- raw-pointer launchers (stream = ctx->stream); validation done by callers
 int zhk_quantize_xq(zh_ctx *ctx, const float *x, void *xq, uint32_t K, uint32_t n_vec,

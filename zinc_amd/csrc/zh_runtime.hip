@@ -58,7 +58,8 @@ extern "C" int zh_init(int device, zh_ctx **out) {
         if (hipEventCreate(&c->ev[i]) != hipSuccess) { delete c; return ZH_ERR_HIP; }
     const uint32_t ctl[2] = {0u, ZH_ATTN_WAIT_TICKS};
     if (hipMalloc((void **)&c->err_dev, 256) != hipSuccess ||
-        hipMemcpy(c->err_dev, ctl, sizeof ctl, hipMemcpyHostToDevice) != hipSuccess) {
+        hipMemcpy(c->err_dev, ctl, sizeof ctl, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMalloc(&c->bmm_ws, ZH_BMM_WS) != hipSuccess) {
         zh_destroy(c);
         return ZH_ERR_HIP;
     }
@@ -71,6 +72,7 @@ extern "C" void zh_destroy(zh_ctx *c) {
     hipSetDevice(c->device);
     hipStreamSynchronize(c->stream);
     if (c->scratch) hipFree(c->scratch);
+    if (c->bmm_ws) hipFree(c->bmm_ws);
     if (c->err_dev) hipFree(c->err_dev);
     for (int i = 0; i < 64; i++) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     hipStreamDestroy(c->stream);

@@ -83,7 +83,7 @@ def test_gemm_matches_fp16_operand_reference(ctx, orc, qtype, M, K, N):
 @pytest.mark.parametrize("qtype,M,K,N", [
     (12, 24500, 512, 509), (12, 24500, 2048, 200),     # 256 tokens x 192 rows, whole and with K split
     (12, 1000, 2304, 129), (14, 1000, 2304, 257), (14, 24500, 256, 256),  # 256 x 128, odd steps, one split
-    (12, 130, 256, 128),                                # 128 x 128
+    (12, 130, 256, 128), (14, 200, 2560, 100),         # 128 x 128
 ])
 def test_gemm_tile_edges(ctx, orc, qtype, M, K, N):
     """Every tile of the dispatch with a ragged last row and token tile,

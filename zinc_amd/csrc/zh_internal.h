@@ -193,7 +193,7 @@ struct zh_gemm_rope {
     uint32_t n_pages, cache_tokens, nq, nkv, pos0;
     float eps;
 };
-// Up to three stacked matrices sharing X (segment rows multiples of 64).
+// Up to three stacked matrices sharing X (rows of all but the last a multiple of 128).
 int zhk_gemm_multi(zh_ctx *ctx, uint32_t qtype, uint32_t nseg, const uint8_t *const *W, const _Float16 *X,
                    uint32_t ldx, float *const *Y, const uint32_t *ldy, const uint32_t *M, uint32_t K, uint32_t N,
                    uint32_t acc, const float *x_unscale = nullptr, const float *norm_w = nullptr,

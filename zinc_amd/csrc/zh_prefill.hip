@@ -461,26 +461,25 @@ int zhk_gemm_multi(zh_ctx *c, uint32_t qtype, uint32_t nseg, const uint8_t *cons
     for (uint32_t s = nseg; s < 3; s++) p.seg_end[s] = end;
     p.M = end;
     for (uint32_t s = 0; s + 1 < nseg; s++)
-        if (M[s] % 64) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "gemm: segment rows %u not a multiple of 64", M[s]);
+        if (M[s] % 128) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "gemm: segment rows %u not a multiple of 128", M[s]);
     // Tile and K split by the time they should take, in K steps of a 256-token
     // x 128-row tile (2.5 us): rounds of workgroups on the device x a
     // workgroup's steps. Measured per step: 1.4 with 192 rows (24576 rows,
     // 1024 tokens: 242 us in two rounds against 266 in three of 128 rows);
-    // 0.65 for a 128-token tile, 0.4 with 64 rows, in CU time (two share a
-    // CU). 96 rows cost a step as long as 128. A launch with fewer tiles than
+    // 0.65 for a 128-token tile, in CU time (two share a CU). 96 rows cost a
+    // step as long as 128. A launch with fewer tiles than
     // fit at once splits K within one round, at least 8 steps per split (the
     // partial sums cost about two steps). 256 tokens from N = 129 on: 24576
     // rows, 129 / 256 / 257 / 512 tokens 71 / 86 / 113 / 125 us against 90 /
-    // 96 / 140 / 163 in 128-token tiles; 4096 rows alike. 64-row tiles only
-    // where a segment boundary needs them.
+    // 96 / 140 / 163 in 128-token tiles; 4096 rows alike.
     const uint32_t cus = (uint32_t)c->cu_count, nst = K / KS;
-    struct { uint32_t ti, tj; float step; } const kinds[] = {{256, 192, 1.4f}, {256, 128, 1.f}, {128, 128, 0.65f}, {128, 64, 0.4f}};
+    struct { uint32_t ti, tj; float step; } const kinds[] = {{256, 192, 1.4f}, {256, 128, 1.f}, {128, 128, 0.65f}};
     uint32_t TI = 0, TJv = 0, ni = 0;
     float best = 0.f;
     for (const auto &k : kinds) {
         bool ok = (k.ti == 128 || N > 128) && (k.tj != 192 || qtype == ZH_Q4_K);
         for (uint32_t s = 0; s + 1 < nseg; s++) ok = ok && M[s] % k.tj == 0;
-        if (!ok || (k.tj == 64 && TI)) continue;
+        if (!ok) continue;
         const uint32_t t = (end + k.tj - 1) / k.tj * ((N + k.ti - 1) / k.ti), slots = k.ti == 256 ? cus : 2 * cus;
         uint32_t sk = t < slots && !zh_knob("ZH_NO_SPLITK") ? slots / t : 1;
         while (sk > 1 && nst < 8 * sk) sk--;
@@ -499,10 +498,9 @@ int zhk_gemm_multi(zh_ctx *c, uint32_t qtype, uint32_t nseg, const uint8_t *cons
     }
     dim3 grid((end + TJv - 1) / TJv, ni, p.ksplit);
 #define GL(Q, J, I) hipLaunchKernelGGL((k_gemm<Q, J, I>), grid, dim3(2 * I), lds, c->stream, p)
-#define GQ(Q)                                     \
-    if (TI == 256 && TJv == 128) GL(Q, 128, 256); \
-    else if (TJv == 128) GL(Q, 128, 128);         \
-    else GL(Q, 64, 128)
+#define GQ(Q)                       \
+    if (TI == 256) GL(Q, 128, 256); \
+    else GL(Q, 128, 128)
     if (TJv == 192) GL(ZH_Q4_K, 192, 256);  // (Q6_K's 96 accumulators and raw bytes do not fit the registers)
     else if (qtype == ZH_Q4_K) { GQ(ZH_Q4_K); }
     else { GQ(ZH_Q6_K); }

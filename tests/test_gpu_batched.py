@@ -178,8 +178,15 @@ def test_batched_allocates_nothing():
     """The first batched calls of 16 contexts leave the device's free memory
     as it is (the operands have a place from the context's creation on, also
     the largest: 16 columns of K = 16384)."""
-    import torch
+    import ctypes as C
     import zinc_amd
+    from zinc_amd.hip import lib
+
+    def free_bytes():  # of the HIP runtime the library runs on
+        free, total = C.c_size_t(), C.c_size_t()
+        assert lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
     M, K, ncol = 256, 16384, 16
     print("batched dmmv allocations", flush=True)
     ctxs = [zinc_amd.Context(0) for _ in range(16)]
@@ -189,11 +196,11 @@ def test_batched_allocates_nothing():
         c.sync()
     ctxs[0].dmmv_batched(12, W, 0, X, 0, Y, 0, M, K, ncol)  # (its code is loaded)
     ctxs[0].sync()
-    free = torch.cuda.mem_get_info()[0]
+    free = free_bytes()
     for c in ctxs[1:]:
         c.dmmv_batched(12, W, 0, X, 0, Y, 0, M, K, ncol)
         c.sync()
-    assert free - torch.cuda.mem_get_info()[0] < 4 << 20  # (the runtime's page granularity is 2 MiB)
+    assert free - free_bytes() < 4 << 20  # (the runtime's page granularity is 2 MiB)
     for b in (W, X, Y):
         ctxs[0].free(b)
     for c in ctxs:

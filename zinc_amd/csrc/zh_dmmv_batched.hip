@@ -416,19 +416,31 @@ static int try_q6k_nv(zh_ctx *c, const LpbP &p, uint32_t nseg, const uint32_t *M
     }
 }
 
-// Whether a launch of 2 or 4 vectors on the tile kernels beats the matrix-unit
-// kernels' two launches (about 8 us together however small the matrix; the
-// tile kernels 5.4 us, but their arithmetic grows with every vector).
-// Measured, tile / matrix units: 2 vectors of Q4_K 4096 x 4096 7.4 / 8.3 us,
-// 1024 x 12288 12.1 / 12.9, 24576 x 2048 9.9 / 12.0, and the other way
-// 24576 x 4096 18.3 / 17.3, 4096 x 12288 19.2 / 13.2; 4 vectors of
-// 4096 x 1024 7.7 / 8.2, and the other way 4096 x 4096 11.0 / 8.4, 24576 x
-// 1024 11.5 / 10.4 us. Q6_K 2048 wide alike (7.9 / 9.2); Q6_K rows
-// of no multiple of 2048 are off the tile kernels. Three vectors are two tile launches (9.3 / 8.1).
-static bool tile_pays(uint32_t nv, uint32_t rows, uint32_t K) {
-    const uint64_t n = (uint64_t)rows * K;
-    if (nv == 2) return K > 4096 ? n < 1ull << 25 : n < 1ull << 26;
-    return nv == 4 && K <= 2048 && rows < 16384;
+// Whether 2 or 4 vectors are faster on the tile kernels than on the matrix
+// units' two launches (about 8 us together however small the matrix). A tile
+// workgroup walks `rounds` batches of 256 / team rows, one after another, and
+// its arithmetic grows with every vector, so what decides is how many rounds.
+// Measured, tile / matrix units:
+//   4 vectors: Q4_K 16384 x 1024 (1 round) 8.1 / 8.5 us, 20480 x 1024 (2)
+//     11.8 / 10.2; gate/up 8192 x 1024 (1) 8.4 / 10.0, 12288 x 1024 (2) 12.6 /
+//     10.1; Q6_K 4096 x 2048 (1) 8.4 / 9.0, 6144 x 2048 (2) 11.0 / 9.4
+//   2 vectors, Q4_K: 49152 x 2048 (6) 17.2 / 19.6, 24576 x 4096 (6) 19.0 /
+//     19.2, 2048 x 8192 (1) 9.7 / 10.4, 3072 x 8192 (2) 12.2 / 10.6
+//   2 vectors, gate/up: 20480 x 2048 (5) 15.1 / 16.9, 6144 x 4096 (3) 12.3 /
+//     13.2, 8192 x 4096 (4) 15.1 / 13.5, 2048 x 8192 (2) 12.6 / 14.4, 1536 x
+//     16384 (3) 20.0 / 22.1, 2048 x 12288 (4) 20.6 / 18.2
+//   2 vectors, Q6_K: 24576 x 2048 (6) 16.1 / 16.7, 6144 x 4096 (3) 11.0 /
+//     13.3, 12288 x 4096 (6) 17.8 / 17.1, 1024 x 12288 (2) 13.4 / 15.3, 2048 x
+//     12288 (4) 17.4 / 16.0
+static bool tile_pays(const zh_ctx *c, uint32_t qtype, int mode, uint32_t nv, uint32_t rows, uint32_t K) {
+    const uint32_t nb = K / 256, lanes = qtype == ZH_Q6_K ? 2 * nb : nb, nm = mode == LPB_GATE_UP ? 2 : 1;
+    const uint32_t rpb = LPB_T / pow2ceil(lanes < 4 ? 4 : lanes) / nm;
+    const uint32_t batches = rpb ? (rows + rpb - 1) / rpb : ~0u, cus = (uint32_t)c->cu_count;
+    const uint32_t rounds = (batches - 1) / cus + 1;
+    if (nv == 4) return K <= 2048 && rounds == 1;
+    if (nv != 2) return false;
+    if (qtype == ZH_Q4_K && mode == LPB_PLAIN) return K <= 4096 || rounds == 1;
+    return K <= 2048 || rounds <= 3;
 }
 
 // Batched DMMV: y[s * n_vec + v] (= or +=) W[s] x_v for v < n_vec, x_v = x[v]
@@ -459,10 +471,10 @@ int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const u
     p.segW2 = W2;
     p.M = end;
     const bool mfma = zhk_dmmv_mfma_fits(qtype, mode, nseg, W, W2, M, K);
-    const uint32_t rows = end * (mode == LPB_GATE_UP ? 2 : 1);
+    const uint32_t nb = K / 256;
     for (uint32_t v0 = 0; v0 < n_vec;) {
         const uint32_t left = n_vec - v0;
-        if (left > 1 && (!mfma || tile_pays(left, rows, K))) {
+        if (left > 1 && (!mfma || tile_pays(c, qtype, mode, left, end, K))) {
             const uint32_t nv = left >= 4 && K <= 2048 ? 4u : 2u;
             LpbB bt = {};
             bt.nv = nv;
@@ -479,8 +491,8 @@ int zhk_dmmv_batched(zh_ctx *c, uint32_t qtype, int mode, uint32_t nseg, const u
             }
         }
         // (two vectors of a small Q6_K matrix off the tile kernels: one by one,
-        // 512 x 512 7.6 us against 9.0)
-        if (mfma && left > 1 && !(left == 2 && tile_pays(2, rows, K))) {
+        // 512 x 512 7.6 us against 9.0, 8192 x 1024 9.1 / 9.3, 4096 x 2304 10.8 / 8.8)
+        if (mfma && left > 1 && !(left == 2 && qtype == ZH_Q6_K && nb % 8 && (uint64_t)end * K < 1u << 23)) {
             const int rc = zhk_dmmv_mfma(c, qtype, mode, nseg, W, W2, M, K, left, x ? x + v0 : nullptr,
                                          x ? nullptr : xq + v0, y + v0, n_vec, norm_w, eps, acc);
             if (rc) return rc;

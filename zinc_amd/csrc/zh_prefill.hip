@@ -901,10 +901,12 @@ int zhk_attn_prefill(zh_ctx *c, const float *q, const uint16_t *kc, const uint16
                      uint32_t N, float scale, _Float16 *out) {
     if (hd != 128 || nkv == 0 || nq % nkv) return zh_set_err(c, ZH_ERR_INVALID_ARGUMENT, "attn_prefill heads");
     const dim3 grid(nq, (N + AQ - 1) / AQ);
-    // two key blocks or fewer for any query: one group, of four waves of 16
+    // three key blocks or fewer for any query: one group, of four waves of 16
     // queries (128 queries at 0: 8.6 us, two waves of 32 9.9, two groups 8.5;
-    // 64: 6.6 / 7.1 / 8.0)
-    if (pos0 + N <= 2 * AK)
+    // 64: 6.6 / 7.1 / 8.0). One group / four: 129 queries at 0 8.8 / 10.5 us,
+    // 192 at 0 10.2 / 11.4, 200 at 0 (four blocks) 11.1 / 11.5, 128 at 128
+    // 12.2 / 11.6, one at 255 10.8 / 9.0
+    if (pos0 + N <= 3 * AK)
         hipLaunchKernelGGL((k_attn_prefill_mfma<1, 1>), grid, dim3(256), AP_GROUP, c->stream, q, kc, vc, pages, n_pages,
                            cache_tokens, nq, nkv, pos0, N, scale, out);
     else

@@ -93,6 +93,42 @@ def test_batch_attention_edges(ctx, n_seq, prefill, heads, paged):
     base.deinit()
 
 
+@pytest.mark.parametrize("n_seq,vocab", [(2, 1000), (5, 1023), (16, 257), (17, 1026)])
+def test_batch_tail(ctx, n_seq, vocab):
+    """Embedding rows, argmax and step advance of up to 16 sequences a launch:
+    vocabularies off the 4 logits of a load and the workgroups of a launch (few
+    and many sequences), a prompt of three tokens, a second run from another
+    position; then logits that are all NaN, whose greedy token is 0, as alone."""
+    import ctypes as C
+    import zinc_amd
+    from zinc_amd.hip import lib
+    print(f"batch tail n={n_seq} vocab {vocab}", flush=True)
+    cfg = dict(CFG, n_layers=1, vocab=vocab, max_ctx=128)
+    base = zinc_amd.InferenceEngine(ctx, cfg)
+    engines = [base] + [base.share(ctx) for _ in range(n_seq - 1)]
+    rng = np.random.default_rng(vocab)
+    for start in (20, 33):
+        prompts = rng.integers(0, vocab, (n_seq, 3)).astype(np.uint32)
+        prompts[0] = [0, vocab - 1, vocab - 1]
+        solo = []
+        for v, e in enumerate(engines):
+            e.prefill_kv_random(start, 500 + v)
+            solo.append(e.generate(prompts[v].tolist(), 5, start_pos=start))
+            e.prefill_kv_random(start, 500 + v)
+        assert zinc_amd.InferenceEngine.generate_batch(engines, prompts, 5, start_pos=start) == solo
+    nan = np.full(cfg["hidden"], np.nan, np.float32)
+    b, off, n = C.c_void_p(), C.c_uint64(), C.c_uint64()
+    ctx.check(lib().zh_engine_tensor(base.h, 2, C.byref(b), C.byref(off), C.byref(n)))  # output_norm
+    assert n.value == nan.nbytes
+    ctx.check(lib().zh_buf_upload(ctx.h, b, off.value, C.c_void_p(nan.ctypes.data), nan.nbytes))
+    got = zinc_amd.InferenceEngine.generate_batch(engines, prompts, 3, start_pos=33)
+    assert got == [[0, 0, 0]] * n_seq
+    assert base.generate(prompts[0].tolist(), 3, start_pos=33) == [0, 0, 0]
+    for e in engines[1:]:
+        e.deinit()
+    base.deinit()
+
+
 @pytest.mark.parametrize("heads", [2, 8, 16])  # 1, 4 and 8 per kv head
 def test_batch_attention_q_past_f16(ctx, heads):
     """Query norm weights of 2^15 put q's components far past f16's 65504:

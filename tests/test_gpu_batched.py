@@ -156,6 +156,32 @@ def test_batched_gate_up_equals_single(ctx, orc, ncol):
         ctx.free(b)
 
 
+@pytest.mark.parametrize("M,nb,ncol", [(1, 1, 2), (129, 2, 5), (70, 5, 9), (34, 9, 16), (300, 15, 13), (4100, 17, 2),
+                                       (50, 33, 16), (30, 49, 8), (46, 48, 12), (18, 64, 3), (34, 64, 16), (520, 64, 7),
+                                       (1030, 16, 9), (10, 65, 2)])
+def test_batched_gate_up_edges(ctx, orc, M, nb, ncol):
+    """Gate and up of different matrices over the row, width (one to four
+    slabs of 16 super-blocks) and group-count classes: silu(g) * u of the two
+    batched DMMVs, which test_batched_edges_equal_single_columns pins, to a few
+    f32 ulps (expf and the division)."""
+    qt, K = 12, 256 * nb
+    print(f"batched gate/up edges {M}x{K} cols {ncol}", flush=True)
+    X = np.stack([orc.synth_normal_f32(K, 96, 10 + v) for v in range(ncol)])
+    Wg, Wu = (ctx.upload(orc.synth_tensor(qt | 0x100, M, K, 95, 1 + m)) for m in range(2))
+    Xb, Yb = ctx.upload(X), ctx.alloc(4 * M * ncol)
+    gu = []
+    for W in (Wg, Wu):
+        ctx.dmmv_batched(qt, W, 0, Xb, 0, Yb, 0, M, K, ncol)
+        gu.append(Yb.download(np.float32, M * ncol))
+    assert not np.array_equal(gu[0], gu[1])
+    ctx.dmmv_fused_gate_up_swiglu_batched(qt, Wg, 0, Wu, 0, Xb, 0, Yb, 0, M, K, ncol)
+    S = Yb.download(np.float32, M * ncol)
+    ref = orc.swiglu(gu[0], gu[1])
+    assert np.allclose(S, ref, rtol=1e-6, atol=1e-7 * np.abs(ref).max()), np.abs(S - ref).max()
+    for b in (Wg, Wu, Xb, Yb):
+        ctx.free(b)
+
+
 def test_batched_rejects_bad_arguments(ctx):
     import zinc_amd
     W, X, Y = ctx.alloc(1 << 22), ctx.alloc(1 << 20), ctx.alloc(1 << 20)

@@ -82,8 +82,10 @@ def test_gemm_matches_fp16_operand_reference(ctx, orc, qtype, M, K, N):
 
 @pytest.mark.parametrize("qtype,M,K,N", [
     (12, 24500, 512, 509), (12, 24500, 2048, 200),     # 256 tokens x 192 rows, whole and with K split
-    (12, 1000, 2304, 129), (14, 1000, 2304, 257), (14, 24500, 256, 256),  # 256 x 128, odd steps, one split
+    (12, 16500, 768, 129), (14, 24500, 256, 256),      # 256 x 128 whole
+    (12, 6100, 2304, 257), (14, 6100, 2304, 257), (14, 3000, 4096, 300),  # with 2 (9 steps each) and 4 splits
     (12, 130, 256, 128), (14, 200, 2560, 100),         # 128 x 128
+    (12, 1000, 2304, 129), (14, 1000, 2304, 257),
 ])
 def test_gemm_tile_edges(ctx, orc, qtype, M, K, N):
     """Every tile of the dispatch with a ragged last row and token tile,
@@ -244,10 +246,11 @@ def test_flash_attn_batched_matches_reference(ctx, nh, nkv, seq_start, n):
 
 @pytest.mark.parametrize("nh,nkv,seq_start,n,scale", [
     (8, 8, 0, 1, 0.0), (8, 1, 63, 1, 0.0), (4, 2, 64, 64, 0.0), (8, 2, 127, 1, 0.0), (8, 2, 128, 1, 0.0),
+    (8, 2, 191, 1, 0.0), (8, 2, 192, 1, 0.0), (4, 2, 0, 192, 0.0), (4, 2, 0, 193, 0.0),
     (4, 4, 65, 63, 0.3), (2, 1, 0, 129, -0.05), (8, 4, 255, 65, 0.0), (16, 2, 500, 200, 0.0)])
 def test_flash_attn_batched_edges(ctx, nh, nkv, seq_start, n, scale):
     """One to thirteen key blocks over the one-group and the four-group form
-    (more than 128 keys), query tiles ending inside one, groups that see no
+    (more than 192 keys), query tiles ending inside one, groups that see no
     key of some queries, every q-per-kv count, a given (also negative) scale.
     The bound of test_flash_attn_batched_matches_reference."""
     rng = np.random.default_rng(nh * 1000 + seq_start + n)
@@ -269,15 +272,15 @@ def test_flash_attn_batched_edges(ctx, nh, nkv, seq_start, n, scale):
 
 
 @pytest.mark.parametrize("cache_tokens", [64, 250])
-@pytest.mark.parametrize("seq_start,n", [(0, 100), (100, 60)])  # the one-group and the four-group form
+@pytest.mark.parametrize("seq_start,n", [(0, 100), (130, 94)])  # the one-group and the four-group form
 def test_flash_attn_batched_page_entries_past_the_cache(ctx, cache_tokens, seq_start, n):
     """A token whose page entry puts it at or past cache_tokens reads cache
     row 0, also where entry * 16 wraps or ends just below 2^32. The bound of
     test_flash_attn_batched_matches_reference."""
     nh, nkv = 4, 2
     rng = np.random.default_rng(cache_tokens + seq_start)
-    pages = np.array([1, 0x0FFFFFFF, 0, cache_tokens // 16, 0xFFFFFFFF, 2, 0x1FFFFFFF, 0x10000001, 3, 0x7FFFFFFF],
-                     np.uint32)
+    pages = np.array([1, 0x0FFFFFFF, 0, cache_tokens // 16, 0xFFFFFFFF, 2, 0x1FFFFFFF, 0x10000001, 3, 0x7FFFFFFF,
+                      0x8FFFFFFF, 2, 0xFFFFFFFE, 1], np.uint32)
     k16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
     v16 = rng.standard_normal((nkv, cache_tokens, 128)).astype(np.float16)
     q = rng.standard_normal((n, nh * 128)).astype(np.float32)

@@ -13,6 +13,7 @@ the group with the largest duration (each runs once per layer, so also the
 largest share of step time).
 
     python -m benchmarks.roofline_probe            # per-kernel table (JSON)
+    python -m benchmarks.roofline_probe --rates    # the card's rates: large copy, read, fp16 product
     rocprofv3 --pmc FETCH_SIZE -- python3 -m benchmarks.roofline_probe --pmc
     rocprofv3 --pmc FETCH_SIZE -- python3 -m benchmarks.roofline_probe --pmc --config 4
 
@@ -77,6 +78,38 @@ def per_kernel(eng, L, iters=108):
     return rows, dom
 
 
+def rates():
+    """What the card reaches on a large copy (bytes read + written), on the
+    library's streaming read, and on a large fp16 matrix product through torch."""
+    import torch  # (before the library's context: torch finds no device once another HIP runtime is up)
+    torch.cuda.init()
+
+    def best(fn, n=20):
+        t = []
+        for _ in range(n):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            fn()
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b) * 1e-3)
+        return min(t)
+    out = {}
+    src = torch.empty(1 << 30, dtype=torch.float32, device="cuda").normal_()
+    dst = torch.empty_like(src)
+    out["copy_4GiB_GBs"] = round(2 * src.numel() * 4 / best(lambda: dst.copy_(src)) / 1e9, 1)
+    for n in (4096, 8192, 16384):
+        x, w = (torch.randn(n, n, dtype=torch.float16, device="cuda") for _ in range(2))
+        y = torch.empty_like(x)
+        out[f"fp16_matmul_{n}_TFLOPs"] = round(2 * n ** 3 / best(lambda: torch.mm(x, w, out=y)) / 1e12, 1)
+    ctx = hip.Context(0)
+    buf = ctx.alloc(4 << 30)
+    ctx.synth_vector(buf, 0, 1, 1 << 31, 1.0, 7, 7)
+    out["stream_read_4GiB_GBs"] = round(ctx.stream_read_probe(buf, 4 << 30, 5), 1)
+    ctx.close()
+    return out
+
+
 def pmc_sequence(ctx, model=DENSE_8B, prefill=PREFILL):
     """Calibration read, calibration write, then every group's launches."""
     cal = ctx.alloc(CAL_BYTES)
@@ -99,7 +132,11 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--pmc", action="store_true", help="run the counter-calibration launch sequence")
     ap.add_argument("--config", type=int, choices=[3, 4], default=3, help="config 3 (dense 8B) or 4 (48-layer MoE)")
+    ap.add_argument("--rates", action="store_true", help="the card's copy, read and matrix-product rates")
     a = ap.parse_args()
+    if a.rates:
+        print(json.dumps(rates()), flush=True)
+        return 0
     model, prefill = (DENSE_8B, PREFILL) if a.config == 3 else (MOE_48L, PREFILL_C4)
     ctx = hip.Context(0)
     if a.pmc:

@@ -327,8 +327,9 @@ int zhk_attn_decode_fused(zh_ctx *c, const float *q, const float *k, const float
 // entry per sequence; the weights and RoPE table are shared. The chunks per
 // kv head shrink with n so that all sequences' chunks fill the device once:
 // with 8 sequences at a 4K context a workgroup streams 1024 tokens (8 x 16.8
-// MB of K/V per layer in 32 us = 4.2 TB/s; the register-pipelined kernel with 22 chunks
-// of 192 tokens per head and sequence, 4 sequences to a launch, took 2 x 31).
+// MB of K/V per layer in 36 us = 3.7 TB/s, the matrix units busy 15% and the
+// VALU 37%; the register-pipelined kernel with 22 chunks of 192 tokens per
+// head and sequence, 4 sequences to a launch, took 2 x 31).
 int zhk_attn_decode_fused_z(zh_ctx *c, uint32_t n, const float *const *q, const float *const *k,
                             const float *const *v, const float *qw, const float *kw, const float *rope_cs,
                             uint16_t *const *kc, uint16_t *const *vc, const uint32_t *const *pages, uint32_t n_pages,

@@ -171,7 +171,9 @@ ZH_DEV void deq_q6k_unit(const RawQ6K &r, uint32_t g, _Float16 *dst) {
 // of the first two per MFMA, so tiles of 256 tokens (half the dequantisation)
 // and 192 rows (1.27 x the MFMAs per LDS byte). 24576 x 4096, 512 tokens: 128
 // x 128 163 us, 256 x 128 155, 256 x 192 125 (826 TFLOP/s); 12288 rows 94 ->
-// 81; Q6_K 4096 x 12288 103 -> 91.
+// 81; Q6_K 4096 x 12288 103 -> 91 (launched without a pause; in short bursts
+// the clock is higher: 146 / 148 / 106, 86 -> 73, 91 -> 83; the weights in the
+// caches or not makes no difference).
 template <int QT, int TJ, int TI>
 __global__ __launch_bounds__(2 * TI, 2) void k_gemm(GemmP p) {
     constexpr int GT = 2 * TI;  // threads: TI / 64 x 2 waves
@@ -654,9 +656,9 @@ __global__ __launch_bounds__(256) void k_swiglu_rows_f16(const float *__restrict
 // blocks g, g + NG, ... of AK = 64 keys, each wave 16 QT queries of them, and the
 // groups' outputs are merged at the end (log-sum-exp weights in LDS). The
 // longest query tile bounds the launch (one workgroup per CU at 512 tokens),
-// so its chain of key blocks is cut by NG. Bound by LDS traffic (1.3 us of
-// the 3.7 a round of NG blocks takes) with the softmax and the MFMAs behind
-// barriers. 32 heads: 512 queries at 0 24 -> 19.4 us, 509 after 1031 tokens
+// so its chain of key blocks is cut by NG. Bound by that chain of loads, LDS
+// round trips, softmax and barriers: of a launch of 512 queries LDS is busy
+// 9%, the VALU 16%, the matrix units 5%. 32 heads: 512 queries at 0 24 -> 19.4 us, 509 after 1031 tokens
 // 66.5 -> 39.7 us (44.5 with four waves of 16 queries per group, which read
 // every K and V fragment twice as often).
 //
@@ -697,7 +699,7 @@ __global__ __launch_bounds__(NG * 256 / QT) void k_attn_prefill_mfma(const float
     const uint32_t i0 = (gridDim.y - 1 - blockIdx.y) * AQ;  // longest tiles first
     const uint16_t *kh = kc + (size_t)kvh * cache_tokens * HD;
     const uint16_t *vh = vc + (size_t)kvh * cache_tokens * HD;
-    // Q fragments (B operand): query i0 + 32 w2 + 16 t + li, d = 32 k4 + 8 lg .. +7
+    // Q fragments (B operand): query i0 + 16 QT w2 + 16 t + li, d = 32 k4 + 8 lg .. +7
     half8 qa[QT][4];
 #pragma unroll
     for (int t = 0; t < QT; t++) {

@@ -385,9 +385,10 @@ ZH_DEV void split_f16(const float (&x)[4], half4 (&h)[N]) {
 // sqrt 2), p by 2^14: three pieces then hold an f32 exactly, less at most
 // 2^-25 of those scaled units, and no q overflows f16. For the batched launch,
 // whose predecessor multiplied in f32. Distance from 64 bits (2-norm, 2 to 4
-// sequences, 32 / 8 heads, f32 kernel / three pieces / two): 4096 tokens 2.1 / 2.0 / 2.8e-7,
-// scores four times as wide 4.9 / 4.8 / 8.4e-7; 16000 tokens 2.4 / 2.1 / 3.2e-7. Eight sequences of 8 layers
-// at 4096 tokens 870 us a step with three pieces, 857 with two.
+// sequences, 32 / 8 heads, f32 kernel / three pieces / two): 4096 tokens 2.1 /
+// 2.0 / 2.8e-7, scores four times as wide 4.9 / 4.8 / 8.4e-7; 16000 tokens 2.4
+// / 2.1 / 3.2e-7. Eight sequences of 8 layers at 4096 tokens: 870 us a step
+// with three pieces, 857 with two.
 constexpr float AR_PSCALE = 16384.f;
 // the exponent field of that power for a head whose largest component is amax
 ZH_DEV uint32_t ar_qscale_field(float amax) {
